@@ -67,6 +67,21 @@ __device__ __forceinline__ double pick(const double* X, int wv)
     }
 }
 
+// n steps of one trajectory, four to a trip: the loop's scalar instructions
+// and taken branch are issue slots to a lone wavefront (LLE preview of 17^2
+// points 403 -> 384 us with the pairs of LleProg::ticks).
+template <class Sy>
+__host__ __device__ __forceinline__ void plain_steps(double* X, const double* a, const StepConst& c, long long n)
+{
+    for (; n >= 4; n -= 4) {
+        Sy::step(X, a, c);
+        Sy::step(X, a, c);
+        Sy::step(X, a, c);
+        Sy::step(X, a, c);
+    }
+    for (; n > 0; --n) Sy::step(X, a, c);
+}
+
 // Lane state parked in HBM between engine launches (SoA, k-major).
 struct LaneStore {
     double* d;     // [nd][np]
@@ -133,7 +148,7 @@ struct LleProg {
         long long g = g0;
         if (g < p.S) {
             const long long e = g1 < p.S ? g1 : p.S;
-            for (long long s = g; s < e; ++s) Sy::step(X, a, p.sc);
+            plain_steps<Sy>(X, a, p.sc, e - g);
             g = e;
         }
         if (g == p.S && g < g1) {
@@ -151,7 +166,14 @@ struct LleProg {
         while (g < g1) {
             const long long left = g1 - g;
             const int n = (p.NTp - local) < left ? (p.NTp - local) : (int)left;  // >= 1: local < NTp
-            for (int s = 0; s < n; ++s) {
+            int s = 0;
+            for (; s + 1 < n; s += 2) {
+                Sy::step(X, a, p.sc);
+                Sy::step(Xp, a, p.sc);
+                Sy::step(X, a, p.sc);
+                Sy::step(Xp, a, p.sc);
+            }
+            if (s < n) {
                 Sy::step(X, a, p.sc);
                 Sy::step(Xp, a, p.sc);
             }
@@ -209,7 +231,7 @@ template <int SYS, int KIND>
 struct SweepProg {
     using Sy = System<SYS>;
     static constexpr int NX = Sy::NX, NA = Sy::NA;
-    static constexpr int ND = NX + 8;  // X, p, dn, first, last, s0, s1, sx, sz
+    static constexpr int ND = NX + 7;  // X, p, first, last, s0, s1, sx, sz
     static constexpr int NI = 4;       // pstart, cnt, prev_t, bits
     double X[NX], a[NA];
     static constexpr bool BIF = stores_peaks(KIND);
@@ -278,64 +300,195 @@ struct SweepProg {
         if (out) alive &= ~wave_mask(lane_bit(out) && diverged_exact(v, A.maxValue, A.check));
     }
 
-    // One recorded sample t: peak detection on the sample, the kind's
-    // per-peak work, then preScaller steps and the divergence check.  BODY:
-    // 2 <= t < B - 1 (detector without the warm-up test, no first/last
-    // sample); PRE1: preScaller == 1.
-    template <int WVT, bool BODY, bool PRE1>
+    // n steps, each followed by the divergence test.  Pairs of steps share one
+    // band test -- the larger magnitude of the two -- and its mask is branched
+    // on after the next pair's steps, as in body().  A NaN stays NaN, so one
+    // that v_max drops from its pair is seen with the next pair or at the end.
+    template <int WVT>
+    __device__ __forceinline__ void checked_steps(const SweepArgs& A, int wv, long long n)
+    {
+        if (n <= 0) return;
+        double v0 = 0.0, v1 = 0.0, m = -1.0;  // no pair yet: inside any band (L >= 0)
+        auto exact = [&](unsigned long long out) {
+            alive &= ~wave_mask(lane_bit(out) && (diverged_exact(v0, A.maxValue, A.check) ||
+                                                  diverged_exact(v1, A.maxValue, A.check)));
+        };
+        auto pair = [&] {
+            const unsigned long long out = wave_mask(!(m < A.L)) & alive;
+            Sy::step(X, a, A.sc);
+            const double w0 = pick<NX, WVT>(X, wv);
+            Sy::step(X, a, A.sc);
+            const double w1 = pick<NX, WVT>(X, wv);
+            pin_state();
+            if (__builtin_expect(out != 0ull, 0)) exact(out);
+            v0 = w0;
+            v1 = w1;
+            m = fmax(fabs(w0), fabs(w1));
+        };
+        for (; n >= 4; n -= 4) {
+            pair();
+            pair();
+        }
+        const unsigned long long out = wave_mask(!(m < A.L)) & alive;
+        if (out) exact(out);
+        for (; n > 0; --n) {
+            Sy::step(X, a, A.sc);
+            check<WVT>(A, wv);
+        }
+        // a NaN of the last pair's second step when no step followed it
+        check<WVT>(A, wv);
+    }
+
+    // The kind's work for the lanes em with a peak (value pv, time pt); em is
+    // wave-uniform and not empty.
+    __device__ __forceinline__ void on_peaks(const SweepArgs& A, WaveCursor& cur, int wave, unsigned long long em,
+                                             double pv, int pt)
+    {
+        const bool e = lane_bit(em);
+        if (BIF) {
+            append_peaks(A.pool, cur, wave, em, pv, pt, cnt);
+            if (e) ++cnt;
+        } else if (KIND == KIND_BASINS_REF) {
+            // running sums of the kept peaks and intervals
+            // (avgPeakFinderCUDA, basinsCUDA.cu:841-861)
+            if (e) {
+                if (cnt >= 1) {
+                    s0 = s0 + pv;
+                    s1 = s1 + (double)(pt - prev_t) * A.hp;
+                }
+                prev_t = pt;
+                ++cnt;
+            }
+        } else {
+            if (e) {
+                if (cnt >= 1) {
+                    s0 = s0 + pv;
+                    s1 = fma(pv, pv, s1);
+                }
+                ++cnt;
+            }
+        }
+    }
+
+    // One recorded sample t at the ends of the record (t < 2, t = B - 1):
+    // peak detection on the sample, the kind's per-peak work, then preScaller
+    // steps and the divergence check.
+    template <int WVT>
     __device__ __forceinline__ void sample(const SweepArgs& A, int wv, WaveCursor& cur, int wave, int t)
     {
         const double v = pick<NX, WVT>(X, wv);
-        if (!BODY && t == 0) first = v;
+        if (t == 0) first = v;
         if (KIND == KIND_BASINS_CFG) {
             sx = sx + X[0];
             sz = sz + X[NX - 1];
         }
         double pv = 0.0;
         int pt = 0;
-        const unsigned long long em = (BODY ? det.feed_body(t - 1, v, pv, pt) : det.feed(t, v, pv, pt)) & alive;
-        const bool e = lane_bit(em);
-        // em is wave-uniform: a wave with no peak at this sample skips the
-        // per-peak work altogether
-        if (em) {
-            if (BIF) {
-                append_peaks(A.pool, cur, wave, em, pv, pt, cnt);
-                if (e) ++cnt;
-            } else if (KIND == KIND_BASINS_REF) {
-                // running sums of the kept peaks and intervals
-                // (avgPeakFinderCUDA, basinsCUDA.cu:841-861)
-                if (e) {
-                    if (cnt >= 1) {
-                        s0 = s0 + pv;
-                        s1 = s1 + (double)(pt - prev_t) * A.hp;
-                    }
-                    prev_t = pt;
-                    ++cnt;
-                }
-            } else {
-                if (e) {
-                    if (cnt >= 1) {
-                        s0 = s0 + pv;
-                        s1 = fma(pv, pv, s1);
-                    }
-                    ++cnt;
-                }
-            }
-        }
-        if (!BODY && t == A.B - 1) {
-            last = v;
-            double xp[NX];
+        const unsigned long long em = det.feed(t, v, pv, pt) & alive;
+        if (em) on_peaks(A, cur, wave, em, pv, pt);
+        double xp[NX];
 #pragma unroll
-            for (int k = 0; k < NX; ++k) xp[k] = X[k];
-            for (int r = 0; r < A.pre; ++r) Sy::step(X, a, A.sc);
-            check<WVT>(A, wv);
+        for (int k = 0; k < NX; ++k) xp[k] = X[k];
+        for (int r = 0; r < A.pre; ++r) Sy::step(X, a, A.sc);
+        check<WVT>(A, wv);
+        if (t == A.B - 1) {
+            last = v;
             fixed = lane_bit(alive) && fixed_point(step_delta2<NX>(X, xp), A.check);
-        } else {
+        }
+    }
+
+    // The value sampled now, added to the sums that every sample feeds.
+    template <int WVT>
+    __device__ __forceinline__ double take(int wv)
+    {
+        if (KIND == KIND_BASINS_CFG) {
+            sx = sx + X[0];
+            sz = sz + X[NX - 1];
+        }
+        return pick<NX, WVT>(X, wv);
+    }
+
+    // Sample t = value v with its masks: divergence first (a value is tested
+    // when it is sampled, which is after the step that made it), then its
+    // peaks.
+    __device__ __forceinline__ void settle(const SweepArgs& A, WaveCursor& cur, int wave, int t, double v,
+                                           unsigned long long c2, unsigned long long tiny, unsigned long long out)
+    {
+        out &= alive;
+        if (out) alive &= ~wave_mask(lane_bit(out) && diverged_exact(v, A.maxValue, A.check));
+        double pv = 0.0;
+        int pt = 0;
+        const unsigned long long em = det.decide(t - 1, v, c2, tiny, pv, pt) & alive;
+        if (em) on_peaks(A, cur, wave, em, pv, pt);
+    }
+
+    // Recorded samples t, t + 1, ... inside the record (2 <= t, t + 1 < end),
+    // two to a trip; returns the first sample not taken.  A peak or a plateau
+    // can only begin where the samples stop rising (up & c2), and the rest of
+    // the detector matters only while a plateau is open or an index is skipped
+    // (busy): one mask says that a pair needs nothing but its steps, and the
+    // divergence band joins it.  The mask is branched on after the second
+    // sample's steps, which do not depend on it (a compare that is branched on
+    // at once stalls a lone wavefront for the time of about six instructions);
+    // the pairs that need no work run in a loop of their own, so that the state
+    // of the detector and of the peak store is not merged back on every trip.
+    // A lone wavefront issues one instruction per 6 clocks whatever its kind,
+    // so fewer scalar instructions and branches a sample count there: the
+    // Rossler diagram of 1000 points 28.9 -> 21.1 ms, BASINS basins of 200^2
+    // 73.5 -> 57.9 ms.  Full grids are bound by FP64 issue and stay (Lorenz
+    // peak map 1024^2 91.4 -> 91.6 ms, basins 1024^2 96.4 -> 95.3 ms).
+    template <int WVT, bool PRE1>
+    __device__ __forceinline__ int body(const SweepArgs& A, int wv, WaveCursor& cur, int wave, int t, int end)
+    {
+        auto advance = [&] {
             if (PRE1) Sy::step(X, a, A.sc);
             else
                 for (int r = 0; r < A.pre; ++r) Sy::step(X, a, A.sc);
-            check<WVT>(A, wv);
+        };
+        unsigned long long busy = det.m.busy();
+        double p = det.p;
+        unsigned long long up = det.m.up;
+        while (t + 1 < end) {
+            double v0, v1;
+            unsigned long long c0, c1, y0, y1, o0, o1, event;
+            do {
+                det.p = p;  // the history before the pair
+                det.m.up = up;
+                v0 = take<WVT>(wv);
+                const double d0 = v0 - p;
+                c0 = wave_mask(d0 <= 0.0);
+                y0 = wave_mask(fabs(d0) <= 1e-13);
+                o0 = wave_mask(!(fabs(v0) < A.L));
+                advance();
+                v1 = take<WVT>(wv);
+                const double d1 = v1 - v0;
+                c1 = wave_mask(d1 <= 0.0);
+                y1 = wave_mask(fabs(d1) <= 1e-13);
+                o1 = wave_mask(!(fabs(v1) < A.L));
+                event = (c0 & up) | (c1 & ~(c0 | y0)) | ((o0 | o1) & alive) | busy;
+                advance();
+                pin_state();
+                t += 2;
+                p = v1;
+                up = ~(c1 | y1);
+            } while (event == 0ull && t + 1 < end);
+            if (event) {
+                settle(A, cur, wave, t - 2, v0, c0, y0, o0);
+                settle(A, cur, wave, t - 1, v1, c1, y1, o1);
+                busy = det.m.busy();
+            }
         }
+        det.p = p;
+        det.m.up = up;
+        check<WVT>(A, wv);  // the last pair's second step
+        return t;
+    }
+
+    // Keeps the steps before this point ahead of the branch that follows.
+    __device__ __forceinline__ void pin_state()
+    {
+#pragma unroll
+        for (int k = 0; k < NX; ++k) asm volatile("" : "+v"(X[k]));
     }
 
     template <int WVT>
@@ -361,10 +514,7 @@ struct SweepProg {
             // fixed point is not recorded and reports 0 (bifurcationCUDA.cu:334-342)
             if (g < A.S - 1) {
                 const long long e = g1 < A.S - 1 ? g1 : A.S - 1;
-                for (long long s = g; s < e; ++s) {
-                    Sy::step(X, a, A.sc);
-                    check<WVT>(A, wv);
-                }
+                checked_steps<WVT>(A, wv, e - g);
                 g = e;
             }
             if (g == A.S - 1 && g < g1) {
@@ -379,7 +529,7 @@ struct SweepProg {
         } else if (g < A.S) {
             // no checks during the Basins transient (basinsCUDA.cu:264-271)
             const long long e = g1 < A.S ? g1 : A.S;
-            for (long long s = g; s < e; ++s) Sy::step(X, a, A.sc);
+            plain_steps<Sy>(X, a, A.sc, e - g);
             g = e;
         }
         // ---- record ----
@@ -388,19 +538,11 @@ struct SweepProg {
         int t = (int)(g - A.S);
         const int te = (int)(g1 - A.S);
         const int body_end = te < B - 1 ? te : B - 1;
-        for (; t < te && t < 2; ++t) sample<WVT, false, false>(A, wv, cur, wave, t);
-        if (A.pre == 1) {
-            // two samples per trip: the detector history and the state
-            // rotate through alternating registers instead of being copied
-            for (; t + 1 < body_end; t += 2) {
-                sample<WVT, true, true>(A, wv, cur, wave, t);
-                sample<WVT, true, true>(A, wv, cur, wave, t + 1);
-            }
-            for (; t < body_end; ++t) sample<WVT, true, true>(A, wv, cur, wave, t);
-        } else {
-            for (; t < body_end; ++t) sample<WVT, true, false>(A, wv, cur, wave, t);
-        }
-        for (; t < te; ++t) sample<WVT, false, false>(A, wv, cur, wave, t);
+        for (; t < te && t < 2; ++t) sample<WVT>(A, wv, cur, wave, t);
+        if (t + 1 < body_end)
+            t = A.pre == 1 ? body<WVT, true>(A, wv, cur, wave, t, body_end)
+                           : body<WVT, false>(A, wv, cur, wave, t, body_end);
+        for (; t < te; ++t) sample<WVT>(A, wv, cur, wave, t);
     }
 
     __device__ __forceinline__ void finish(const SweepArgs& A, long long q) const
@@ -469,21 +611,21 @@ struct SweepProg {
         for (int k = 0; k < NX; ++k) X[k] = L.d[k * L.np + q];
         const double* d = L.d + NX * L.np + q;
         det.p = d[0];
-        det.dn = d[L.np];
-        first = d[2 * L.np];
-        last = d[3 * L.np];
-        s0 = d[4 * L.np];
-        s1 = d[5 * L.np];
-        sx = d[6 * L.np];
-        sz = d[7 * L.np];
+        first = d[L.np];
+        last = d[2 * L.np];
+        s0 = d[3 * L.np];
+        s1 = d[4 * L.np];
+        sx = d[5 * L.np];
+        sz = d[6 * L.np];
         det.pstart = L.i[q];
         cnt = L.i[L.np + q];
         prev_t = L.i[2 * L.np + q];
         const int bits = L.i[3 * L.np + q];
         alive = wave_mask(bits & 1);
         fixed = bits & 2;
-        det.plat = wave_mask(bits & 4);
-        det.skip = wave_mask(bits & 8);
+        det.m.plat = wave_mask(bits & 4);
+        det.m.skip = wave_mask(bits & 8);
+        det.m.up = wave_mask(bits & 16);
     }
     __device__ __forceinline__ void store(const LaneStore& L, long long q) const
     {
@@ -491,18 +633,18 @@ struct SweepProg {
         for (int k = 0; k < NX; ++k) L.d[k * L.np + q] = X[k];
         double* d = L.d + NX * L.np + q;
         d[0] = det.p;
-        d[L.np] = det.dn;
-        d[2 * L.np] = first;
-        d[3 * L.np] = last;
-        d[4 * L.np] = s0;
-        d[5 * L.np] = s1;
-        d[6 * L.np] = sx;
-        d[7 * L.np] = sz;
+        d[L.np] = first;
+        d[2 * L.np] = last;
+        d[3 * L.np] = s0;
+        d[4 * L.np] = s1;
+        d[5 * L.np] = sx;
+        d[6 * L.np] = sz;
         L.i[q] = det.pstart;
         L.i[L.np + q] = cnt;
         L.i[2 * L.np + q] = prev_t;
         L.i[3 * L.np + q] =
-            (lane_bit(alive) ? 1 : 0) | (fixed ? 2 : 0) | (lane_bit(det.plat) ? 4 : 0) | (lane_bit(det.skip) ? 8 : 0);
+            (lane_bit(alive) ? 1 : 0) | (fixed ? 2 : 0) | (lane_bit(det.m.plat) ? 4 : 0) |
+            (lane_bit(det.m.skip) ? 8 : 0) | (lane_bit(det.m.up) ? 16 : 0);
     }
 };
 

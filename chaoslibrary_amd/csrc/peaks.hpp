@@ -109,67 +109,90 @@ struct PeakDetector {
 __device__ __forceinline__ unsigned long long wave_mask(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 __device__ __forceinline__ bool lane_bit(unsigned long long m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
-// PeakDetector for a whole wave, as the sweeps use it: the same transitions
-// with the two state flags held as wave masks (SGPRs).  The three tests are
-// compares written into masks, the state machine runs on the scalar unit and
-// the emit mask feeds the wave's append directly -- a per-lane bool state
-// costs two VALU instructions per sample to form each ballot.  All 64 lanes
-// must take every call (wave-uniform control flow).  TIMES: track the
-// plateau start and report peak times (not needed when only peak values are
-// used).
-template <bool TIMES>
-struct WavePeakDetector {
-    double p;                 // last sample d[t-1]
-    double dn;                // d[t-1] - d[t-2]
-    int pstart;               // plateau start index
+// PeakDetector's state for a whole wave as lane masks (SGPRs).  With
+// dnx = d[t] - d[t-1], two compares a sample give all three tests: c2 =
+// (dnx <= 0) and tiny = (|dnx| <= 1e-13), for d[c] - d[c+1] > 1e-13 is
+// c2 & ~tiny, and the rising test of the next sample, dn > 1e-13, is
+// ~(c2 | tiny).  (Of a NaN difference both compares are false; the next
+// difference is NaN too, so no candidate comes of it.)  The state machine runs
+// on the scalar unit -- a per-lane bool state costs two VALU instructions per
+// sample to form each ballot.
+struct PeakMasks {
+    unsigned long long up;    // lanes with d[t-1] - d[t-2] > 1e-13
     unsigned long long plat;  // lanes scanning a plateau
     unsigned long long skip;  // lanes whose next index is not a candidate
+
+    struct Found {
+        unsigned long long emit;    // lanes with a peak at c = t - 1
+        unsigned long long closed;  // of them, those that end a plateau
+        unsigned long long opened;  // lanes that begin a plateau at c
+    };
+
+    // PeakDetector::feed_body for every lane (t >= 2).  skip is kept only
+    // where it matters, after a plateau that rose again: after a peak
+    // dnx < -1e-13, so the next index fails its own rising test.  So with
+    // no plateau open and nothing skipped (quiet), a sample finds no peak and
+    // opens no plateau unless up & c2.
+    __host__ __device__ __forceinline__ Found step(unsigned long long c2, unsigned long long tiny)
+    {
+        const unsigned long long c3 = c2 & ~tiny;
+        const unsigned long long cand = ~plat & ~skip & up & c2;
+        const unsigned long long act = plat | cand;
+        const Found f = {act & c3, plat & c3, cand & ~c3};
+        skip = plat & ~c2;
+        plat = act & c2 & tiny;
+        up = ~(c2 | tiny);
+        return f;
+    }
+    __host__ __device__ __forceinline__ unsigned long long busy() const { return plat | skip; }
+};
+
+// PeakDetector for a whole wave, as the sweeps use it: the masks, the last
+// sample's value and the plateau starts.  The compares are written into masks
+// and the emit mask feeds the wave's append directly.  All 64 lanes must take
+// every call (wave-uniform control flow).  TIMES: track the plateau start and
+// report peak times (not needed when only peak values are used).
+template <bool TIMES>
+struct WavePeakDetector {
+    double p;    // last sample d[t-1]
+    int pstart;  // plateau start index
+    PeakMasks m;
 
     __device__ __forceinline__ void reset()
     {
         p = 0.0;
-        dn = 0.0;
         pstart = 0;
-        plat = 0ull;
-        skip = 0ull;
+        m.up = m.plat = m.skip = 0ull;
     }
 
-    // t >= 2, c = t - 1: PeakDetector::feed_body over the wave; returns the
-    // mask of lanes with a peak at c (value val, time time).
-    __device__ __forceinline__ unsigned long long feed_body(int c, double cur, double& val, int& time)
+    // t >= 2, c = t - 1: the sample cur with its masks c2 and tiny; returns
+    // the mask of lanes with a peak at c (value val, time time).
+    __device__ __forceinline__ unsigned long long decide(int c, double cur, unsigned long long c2,
+                                                         unsigned long long tiny, double& val, int& time)
     {
-        const double dnx = cur - p;
-        const unsigned long long c1 = wave_mask(dn > 1e-13);
-        const unsigned long long c2 = wave_mask(dnx <= 0.0);
-        const unsigned long long c3 = wave_mask(dnx < -1e-13);
-        const unsigned long long cand = ~plat & ~skip & c1 & c2;
-        const unsigned long long act = plat | cand;
-        const unsigned long long emit = act & c3;
-        const unsigned long long flat = c2 & ~c3;
+        const unsigned long long plat = m.plat;
+        const PeakMasks::Found f = m.step(c2, tiny);
         val = p;
+        time = 0;
         if (TIMES) {
             // a peak's time is its sample index, or the middle of the
             // plateau for a lane that ends one; plateaus are rare, so both
             // lane updates sit behind wave-uniform branches
             time = c;
-            if (plat & c3) time = lane_bit(plat) ? (pstart + c) >> 1 : c;
-            const unsigned long long ps = cand & flat;
-            if (ps) pstart = lane_bit(ps) ? c : pstart;
-        } else {
-            time = 0;
+            if (f.closed) time = lane_bit(plat) ? (pstart + c) >> 1 : c;
+            if (f.opened) pstart = lane_bit(f.opened) ? c : pstart;
         }
-        skip = (plat & ~flat) | (cand & c3);
-        plat = act & flat;
-        dn = dnx;
         p = cur;
-        return emit;
+        return f.emit;
     }
 
-    // Any t: samples 0 and 1 only fill the history.
+    // Any t: sample 0 only fills the history, sample 1 only the rising test.
     __device__ __forceinline__ unsigned long long feed(int t, double cur, double& val, int& time)
     {
-        if (t >= 2) return feed_body(t - 1, cur, val, time);
-        dn = cur - p;
+        const double dnx = cur - p;
+        const unsigned long long c2 = wave_mask(dnx <= 0.0), tiny = wave_mask(fabs(dnx) <= 1e-13);
+        if (t >= 2) return decide(t - 1, cur, c2, tiny, val, time);
+        m.up = ~(c2 | tiny);
         p = cur;
         val = 0.0;
         time = 0;
@@ -245,9 +268,13 @@ __device__ __forceinline__ void append_peaks(const PeakPool& pool, WaveCursor& c
         cur.chunk = nc;
         cur.fill = 0;
     }
+    // the cursor moves on before the divergent store, which keeps it in SGPRs
+    // (moved after it, it is merged from both sides of the store's condition)
+    const unsigned base_fill = (unsigned)cur.fill;
+    cur.fill += n;
     if (emit && cur.chunk < pool.nchunks) {
         // wave-uniform chunk base + a 32-bit byte offset inside the chunk
-        const unsigned off = ((unsigned)cur.fill + lane_prefix(m)) * (unsigned)sizeof(PeakEntry);
+        const unsigned off = (base_fill + lane_prefix(m)) * (unsigned)sizeof(PeakEntry);
         char* base = (char*)(pool.entries + (size_t)cur.chunk * kChunk);
         PeakEntry e;
         e.v = v;
@@ -255,7 +282,6 @@ __device__ __forceinline__ void append_peaks(const PeakPool& pool, WaveCursor& c
         e.kl = ((unsigned)k << 6) | (unsigned)__lane_id();
         *(PeakEntry*)(base + off) = e;
     }
-    cur.fill += n;
 }
 
 }  // namespace chaos
