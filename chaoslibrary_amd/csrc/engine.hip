@@ -69,37 +69,6 @@ __device__ __forceinline__ void lle_group(const JobDev& J, const Tile& T, long l
     }
 }
 
-// One 64-point group of a sweep job; WV is the recorded variable.
-template <int SYS, int KIND, int WV>
-__device__ __forceinline__ void sweep_group(const JobDev& J, const Tile& T, long long group, int lane)
-{
-    const SweepArgs& A = J.sw;
-    const long long q = group * 64 + lane;
-    const bool in_range = q < A.n_points;
-    const long long qq = in_range ? q : 0;
-    SweepProg<SYS, KIND> L;
-    WaveCursor cur{A.pool.nchunks, kChunk};
-    if (T.g0 == 0) {
-        L.init(A, qq, in_range);
-    } else {
-        L.params(A, qq);
-        L.load(J.st, q);
-        if (KIND == KIND_BIF) {
-            const WaveCursor c = J.cursors[group];
-            cur.chunk = __builtin_amdgcn_readfirstlane(c.chunk);
-            cur.fill = __builtin_amdgcn_readfirstlane(c.fill);
-        }
-    }
-    L.template ticks<WV>(A, WV, cur, (int)group, T.g0, T.g1);
-    if (T.g1 == J.total) {
-        if (KIND == KIND_BIF) close_chunk(A.pool, cur);
-        if (in_range) L.finish(A, q);
-    } else {
-        L.store(J.st, q);
-        if (KIND == KIND_BIF && lane == 0) J.cursors[group] = cur;
-    }
-}
-
 // Tile checks shared by the families: the tile's job must be of the
 // kernel's family, its tick range inside [0, total] and its groups inside
 // the job.  A failed check sets an error bit and skips the tile; the host
@@ -163,7 +132,7 @@ void engine_sweep_kernel(const JobDev* __restrict__ jobs, const Tile* __restrict
     drain_family(tiles, ctl, FAM, [&](const Tile& T, int lane) {
         const JobDev& J = jobs[T.slot];
         if (!tile_ok(J, T, FAM, &ctl->err)) return;
-        sweep_group<SYS, KIND, WV>(J, T, T.group, lane);
+        sweep_group_ticks<SYS, KIND, WV>(J.sw, J.st, J.cursors, J.total, T.group, lane, T.g0, T.g1);
     });
 }
 

@@ -648,4 +648,39 @@ struct SweepProg {
     }
 };
 
+// Ticks [g0, g1) of one 64-point group of a sweep whose lane state is parked in
+// st (and, for the kinds that store peaks, its peak-store cursor in cursors)
+// between calls; writes the outputs when g1 is the last tick.  All 64 lanes of
+// the wave call it.
+template <int SYS, int KIND, int WV>
+__device__ __forceinline__ void sweep_group_ticks(const SweepArgs& A, const LaneStore& st, WaveCursor* cursors,
+                                                  long long total, long long group, int lane, long long g0,
+                                                  long long g1)
+{
+    const long long q = group * 64 + lane;
+    const bool in_range = q < A.n_points;
+    const long long pq = A.p0 + (in_range ? q : 0);
+    SweepProg<SYS, KIND> L;
+    WaveCursor cur{A.pool.nchunks, kChunk};
+    if (g0 == 0) {
+        L.init(A, pq, in_range);
+    } else {
+        L.params(A, pq);
+        L.load(st, q);
+        if (stores_peaks(KIND)) {
+            const WaveCursor c = cursors[group];
+            cur.chunk = __builtin_amdgcn_readfirstlane(c.chunk);
+            cur.fill = __builtin_amdgcn_readfirstlane(c.fill);
+        }
+    }
+    L.template ticks<WV>(A, WV, cur, (int)group, g0, g1);
+    if (g1 == total) {
+        if (stores_peaks(KIND)) close_chunk(A.pool, cur);
+        if (in_range) L.finish(A, q);
+    } else {
+        L.store(st, q);
+        if (stores_peaks(KIND) && lane == 0) cursors[group] = cur;
+    }
+}
+
 }  // namespace chaos

@@ -1,0 +1,86 @@
+// rotate.hpp -- wavefronts of one launch taking turns on the SIMDs.
+//
+// A grid of, say, 1.4 wavefronts per SIMD launched at once leaves most SIMDs
+// one wavefront and some two, and ends when those two do.  A rotating launch
+// starts a whole number of wavefronts per SIMD; each takes the next ticket of
+// the run (chunk c of group g is ticket c * groups + g), loads the group's lane
+// state, advances it over the chunk's ticks and parks it again.  The lane
+// programs give the same bits however their ticks are cut.  rotate_plan.hpp
+// says when this is used and what it measured.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "runtime.hpp"
+
+namespace chaos {
+
+// Device control block: the ticket counter, an error word and, per group, the
+// chunks done.
+struct RotateCtl {
+    unsigned* head;
+    int* err;
+    unsigned* done;  // [groups]
+    unsigned groups;
+    unsigned chunks;
+};
+
+// Polls of a wait before it is given up (a poll takes about a microsecond).
+constexpr unsigned kRotatePolls = 1u << 27;
+
+// body(group, chunk, lane) for every ticket.  A ticket's predecessor (the same
+// group's chunk before it) was handed out earlier, to a wavefront that is
+// running -- only running wavefronts take tickets -- and each holds one ticket
+// at a time, so the wait for it ends; every wavefront leaves when the tickets
+// are used up.  A wait that does not end all the same is given up after
+// kRotatePolls: the error word is set, the wavefront leaves, and the host
+// reports the call as failed.  The state crosses the XCDs' L2 caches between
+// chunks: parked and released at agent scope, acquired before it is loaded.
+//
+// The ticket is read from the first active lane, so the lanes must come to it
+// together: every trip ends in a wave barrier, which keeps lanes that skip a
+// divergent tail of the body (or of the hand-over) from taking the back edge on
+// their own.
+template <class Body>
+__device__ __forceinline__ void rotate(const RotateCtl& ctl, Body&& body)
+{
+    const int lane = threadIdx.x & 63;
+    const unsigned total = ctl.groups * ctl.chunks;
+    for (unsigned trip = 0; trip <= total; ++trip) {
+        // one ticket a wave: its 64 lanes add 1 each (one atomic of 64), the
+        // first lane gets the sum before them
+        const unsigned t = __builtin_amdgcn_readfirstlane(atomicAdd(ctl.head, 1u)) >> 6;
+        if (t >= total) break;
+        const unsigned c = t / ctl.groups, g = t - c * ctl.groups;
+        if (c > 0) {
+            unsigned polls = 0;
+            while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(&ctl.done[g], __ATOMIC_RELAXED,
+                                                                    __HIP_MEMORY_SCOPE_AGENT)) < c &&
+                   ++polls < kRotatePolls)
+                __builtin_amdgcn_s_sleep(16);
+            if (polls == kRotatePolls) {
+                __hip_atomic_store(ctl.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        }
+        body(g, c, lane);
+        __builtin_amdgcn_wave_barrier();
+        if (c + 1 < ctl.chunks) {
+            // every lane stores the same word: no divergent branch
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            __hip_atomic_store(&ctl.done[g], c + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// Control block in call scratch, cleared on the call's stream (a kernel, not a
+// memset); its error word is checked when the call finishes.
+RotateCtl make_rotate_ctl(CallCtx& ctx, long long groups, long long chunks);
+// Blocks of 256 threads that put `waves` wavefronts on every SIMD.
+unsigned rotate_grid(CallCtx& ctx, int waves);
+// SIMDs of the call's device (four per CU).
+long long device_simds(CallCtx& ctx);
+
+}  // namespace chaos

@@ -1,0 +1,61 @@
+// rotate_plan.hpp -- when a grid's wavefronts take turns on the SIMDs, as
+// plain host C++ (no HIP types), so that it runs and is tested on machines
+// without a GPU.
+#pragma once
+
+namespace chaos {
+
+// The two kinds of per-lane program: exponent maps (two trajectories, no
+// per-sample work: two wavefronts on a SIMD already fill its FP64 unit) and
+// sweeps (per-sample scalar work and branches, which more wavefronts hide).
+enum RotateKind { ROTATE_LLE, ROTATE_SWEEP };
+
+constexpr long long kRotateChunk = 2000;  // fewest ticks per chunk
+constexpr int kRotateMinChunks = 12, kRotateMaxChunks = 48;
+
+// Wavefronts per SIMD of a rotating launch (rotate.hpp) over `groups`
+// wavefronts of work, or 0 to launch them all at once.
+//
+// At once, the SIMDs that hold ceil(w) wavefronts (w = groups / simds) finish
+// last and the others idle meanwhile; rotating, simds * k wavefronts take the
+// groups' chunks in turn and every SIMD does w of the work.  In units of a
+// wavefront's share of a full SIMD the times were, on 1024 SIMDs over w = 1 to
+// 8 (Rossler, Lorenz and Chameleon maps of 258^2 to 720^2 points, 80,000 and
+// 60,000 ticks):
+//   exponent maps: at once ceil(w); k = 1: 1.03 w; k = 2: 0.92 w + 0.6
+//   sweeps:        at once ceil(w) + 0.34; k = 1: 1.33 w; k = 2: w + 0.38
+// (with k = 2 a chunk's predecessor has only just finished when w is little
+// above 2, and k = 3 or 4 were never ahead).  For instance, at once / rotating:
+// Rossler exponents 258^2 (w = 1.02) 18.7 / 9.7 ms, 300^2 (1.37) 17.2 / 12.7,
+// 400^2 (2.44) 26.7 / 22.1, 600^2 (5.49) 52.8 / 49.6; Lorenz peak map 300^2
+// 13.6 / 11.5, 400^2 19.7 / 16.4, 600^2 36.5 / 33.8; Chameleon peak map 300^2
+// 16.4 / 13.3.  The plain launch stays where it is within 2 %, above eight
+// wavefronts a SIMD (the most that reside: the hardware's refill evens the
+// load), and for runs of fewer than 12 chunks of 2000 ticks (`ticks` per
+// group): shorter chunks cost too much to hand over and fewer leave an uneven
+// end of their own.
+inline int rotate_waves(RotateKind kind, long long groups, long long simds, long long ticks)
+{
+    if (simds <= 0 || groups <= simds || groups > 8 * simds) return 0;
+    if (ticks < kRotateChunk * kRotateMinChunks) return 0;
+    const double w = (double)groups / (double)simds;
+    const double c = (double)((groups + simds - 1) / simds);
+    const double at_once = kind == ROTATE_LLE ? c : c + 0.34;
+    const double one = kind == ROTATE_LLE ? 1.03 * w : 1.33 * w;
+    const double two = groups < 2 * simds ? 1e30 : kind == ROTATE_LLE ? 0.92 * w + 0.6 : w + 0.38;
+    const double best = one < two ? one : two;
+    if (best >= 0.98 * at_once) return 0;
+    return one < two ? 1 : 2;
+}
+
+// Ticks per chunk: a run of `ticks` in at most kRotateMaxChunks chunks of at
+// least kRotateChunk ticks, rounded up to a multiple of `unit`.
+inline long long rotate_chunk_ticks(long long ticks, long long unit)
+{
+    long long c = (ticks + kRotateMaxChunks - 1) / kRotateMaxChunks;
+    if (c < kRotateChunk) c = kRotateChunk;
+    if (unit < 1) unit = 1;
+    return (c + unit - 1) / unit * unit;
+}
+
+}  // namespace chaos

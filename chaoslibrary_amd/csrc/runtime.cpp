@@ -250,8 +250,28 @@ CallCtx::CallCtx(const chaos_options& o, bool library_stream_ok) : opt_(o), devi
     stream_ = o.stream ? static_cast<hipStream_t>(o.stream) : (library_stream_ok ? library_stream(device_) : nullptr);
 }
 
+void* CallCtx::scratch(ScratchSlot slot, size_t bytes)
+{
+    if (bytes > scratch_bytes_[slot]) {
+        if (scratch_[slot]) {
+            sync();
+            dev_free(scratch_[slot]);
+            scratch_[slot] = nullptr;
+            scratch_bytes_[slot] = 0;
+        }
+        scratch_[slot] = dev_alloc(bytes);
+        scratch_bytes_[slot] = bytes;
+    }
+    return scratch_[slot];
+}
+
 CallCtx::~CallCtx()
 {
+    bool any = false;
+    for (void* p : scratch_) any = any || p;
+    if (any) (void)hipStreamSynchronize(stream_);
+    for (void* p : scratch_)
+        if (p) dev_free(p);
     if (ev0_) (void)hipEventDestroy(ev0_);
     if (ev1_) (void)hipEventDestroy(ev1_);
     (void)hipSetDevice(prev_device_);
@@ -277,8 +297,19 @@ double CallCtx::end()
 
 void CallCtx::sync() { CHAOS_HIP(hipStreamSynchronize(stream_)); }
 
+void CallCtx::check_watched()
+{
+    if (!watched_) return;
+    int v = 0;
+    CHAOS_HIP(hipMemcpyAsync(&v, watched_, sizeof v, hipMemcpyDeviceToHost, stream_));
+    sync();
+    watched_ = nullptr;
+    if (v != 0) fail(CHAOS_E_HIP, "a launch gave up waiting for a part of its own work (device error word %d)", v);
+}
+
 void CallCtx::finish()
 {
+    check_watched();
     if (!opt_.stats) return;
     chaos_stats* s = opt_.stats;
     s->kernel_ms = kernel_ms_;

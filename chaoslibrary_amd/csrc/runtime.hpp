@@ -133,11 +133,21 @@ public:
     void begin();
     double end();            // returns ms of this region (synchronises)
     void sync();
+    // Device scratch of the call's launches, one block per slot: kept for the
+    // call's next launch (its launches follow each other on one stream), grown
+    // when that needs more, freed with the context after its stream is idle.
+    enum ScratchSlot { SCRATCH_CTL, SCRATCH_STATE, SCRATCH_INTS, SCRATCH_CURSORS, SCRATCH_SLOTS };
+    void* scratch(ScratchSlot slot, size_t bytes);
     void add_kernel_ms(double ms) { kernel_ms_ += ms; }
     void add_analysis_ms(double ms) { analysis_ms_ += ms; }
     void add_steps(double s) { steps_ += s; }
     void add_launch(int n = 1) { launches_ += n; }
     void add_peaks(long long n) { peaks_ += n; }
+    // A device error word of the launches so far: finish() fails the call when
+    // it is not 0 (the word must live as long as the context; check_watched()
+    // reads it now, before the word is used anew).
+    void watch(const int* word) { watched_ = word; }
+    void check_watched();
     void finish();          // fill opt.stats
 
 private:
@@ -150,6 +160,9 @@ private:
     long long peaks_ = 0;
     int launches_ = 0;
     double t0_ = 0;
+    const int* watched_ = nullptr;
+    void* scratch_[SCRATCH_SLOTS] = {};
+    size_t scratch_bytes_[SCRATCH_SLOTS] = {};
 };
 
 double wall_ms();

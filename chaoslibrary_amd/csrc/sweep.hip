@@ -15,6 +15,8 @@
 #include "dispatch.hpp"
 #include "lanes.hpp"
 #include "moments.hpp"
+#include "rotate.hpp"
+#include "rotate_plan.hpp"
 #include "sweep.hpp"
 
 namespace chaos {
@@ -78,6 +80,11 @@ void launch_sweep(CallCtx& ctx, int system, int writableVar, int kind, const Swe
     int nx = 0, na = 0;
     chaos_system_dims(system, &nx, &na);
     CHAOS_REQUIRE(writableVar >= 0 && writableVar < nx, "writableVar %d out of range [0,%d)", writableVar, nx);
+    if (const int turn = rotate_waves(ROTATE_SWEEP, ceil_div((unsigned long long)A.n_points, 64), device_simds(ctx),
+                                      (long long)A.S + A.B)) {
+        launch_sweep_rotating(ctx, system, writableVar, kind, A, turn);
+        return;
+    }
     dispatch_system(system, [&](auto tag) {
         constexpr int S = decltype(tag)::value;
         constexpr int NXs = System<S>::NX;

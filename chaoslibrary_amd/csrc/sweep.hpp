@@ -63,6 +63,10 @@ struct SweepArgs {
 // Fast-path bound for the divergence test of each check mode.
 double divergence_fast_bound(int check, double maxValue);
 
+// The sweep with its wavefronts taking turns, `waves` of them on every SIMD
+// (rotate_plan.hpp); launch_sweep picks it.
+void launch_sweep_rotating(CallCtx& ctx, int system, int writableVar, int kind, const SweepArgs& A, int waves);
+
 void launch_sweep(CallCtx& ctx, int system, int writableVar, int kind, const SweepArgs& A);
 
 }  // namespace chaos
