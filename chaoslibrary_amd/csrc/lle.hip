@@ -64,6 +64,132 @@ void lle_rotate_kernel(const LleArgs p, const RotateCtl ctl, long long chunk, co
     });
 }
 
+// The transient alone, one lane per point; X to xs[k * xn + q].
+template <int SYS>
+__global__ __launch_bounds__(256) void lle_transient_kernel(const LleArgs p, double* __restrict__ xs, long long xn)
+{
+    using P = LleProg<SYS>;
+    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= p.n_points) return;
+    P L;
+    L.params(p, (int)(q % p.nPts), (int)(p.row0 + q / p.nPts));
+    L.init(p);
+    plain_steps<typename P::Sy>(L.X, L.a, p.sc, p.S);
+#pragma unroll
+    for (int k = 0; k < P::NX; ++k) xs[k * xn + q] = L.X[k];
+}
+
+// The other lane's value of an even / odd lane pair.
+__device__ __forceinline__ double pair_swap(double v)
+{
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0xB1, 0xF, 0xF, true);  // quad_perm [1,0,3,2]
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0xB1, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+
+// Windows [w0, w1) of a point on a lane pair: the even lane steps X, the odd
+// lane Xp, in T; each window ends with LleProg::ticks' renormalisation, done
+// on both lanes from the same difference (the odd lane has its negative, which
+// rounds alike) and applied by the odd one.
+template <int SYS>
+__device__ __forceinline__ void pair_windows(const LleArgs& p, const double* a, bool odd, double* T, double& sum,
+                                             int w0, int w1)
+{
+    using Sy = System<SYS>;
+    constexpr int NX = Sy::NX;
+    for (int w = w0; w < w1; ++w) {
+        plain_steps<Sy>(T, a, p.sc, p.NTp);
+        double o[NX], e[NX], d2 = 0.0;
+#pragma unroll
+        for (int l = 0; l < NX; ++l) {
+            o[l] = pair_swap(T[l]);
+            e[l] = o[l] - T[l];
+            d2 = d2 + e[l] * e[l];
+        }
+        const double dist = sqrt(d2) / p.eps;
+        sum = sum + log(dist);
+#pragma unroll
+        for (int l = 0; l < NX; ++l) {
+            const double r = o[l] - e[l] / dist;  // on the odd lane: X - (X - Xp) / dist
+            T[l] = odd ? r : T[l];
+        }
+    }
+}
+
+// The Benettin windows with a point's two trajectories on two neighbouring
+// lanes (lle_split): for grids that leave SIMDs without a wavefront, where the
+// time of a tick is its instructions.  xs: the states after the transient, or
+// NULL when there was none.  Rossler preview of 17^2 points 384 -> 251 us,
+// Chameleon map of 200^2 23.1 -> 20.7 ms.
+template <int SYS>
+__device__ __forceinline__ void pair_begin(const LleArgs& p, long long q, bool odd, const double* xs, long long xn,
+                                           double* a, double* T)
+{
+    using P = LleProg<SYS>;
+    P L;
+    const int i = (int)(q % p.nPts), j = (int)(p.row0 + q / p.nPts);
+    L.params(p, i, j);
+#pragma unroll
+    for (int k = 0; k < P::NA; ++k) a[k] = L.a[k];
+    if (T == nullptr) return;
+    double d[P::NX];
+    P::offset(p, (long long)j * p.nPts + i, d);
+#pragma unroll
+    for (int k = 0; k < P::NX; ++k) {
+        const double x = xs ? xs[k * xn + q] : p.ic[k];
+        T[k] = odd ? x + d[k] : x;
+    }
+}
+
+template <int SYS>
+__global__ __launch_bounds__(256) void lle_pair_kernel(const LleArgs p, const double* __restrict__ xs, long long xn,
+                                                       double* __restrict__ out)
+{
+    using P = LleProg<SYS>;
+    const long long h = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long q = h >> 1;
+    if (q >= p.n_points) return;
+    const bool odd = h & 1;
+    double a[P::NA], T[P::NX], sum = 0.0;
+    pair_begin<SYS>(p, q, odd, xs, xn, a, T);
+    pair_windows<SYS>(p, a, odd, T, sum, 0, p.W);
+    if (!odd) out[q] = sum / p.tMax;
+}
+
+// The same with the wavefronts taking turns: groups of 32 points, chunks of
+// `chunk` windows.
+template <int SYS>
+__global__ __launch_bounds__(256) void lle_pair_rotate_kernel(const LleArgs p, const RotateCtl ctl, int chunk,
+                                                              const double* __restrict__ xs, long long xn,
+                                                              const LaneStore st, double* __restrict__ out)
+{
+    using P = LleProg<SYS>;
+    rotate(ctl, [&](unsigned g, unsigned c, int lane) {
+        const long long h = (long long)g * 64 + lane;
+        const long long q = (h >> 1) < p.n_points ? h >> 1 : 0;
+        const bool odd = h & 1;
+        double a[P::NA], T[P::NX], sum = 0.0;
+        if (c == 0) {
+            pair_begin<SYS>(p, q, odd, xs, xn, a, T);
+        } else {
+            pair_begin<SYS>(p, q, odd, xs, xn, a, nullptr);
+#pragma unroll
+            for (int k = 0; k < P::NX; ++k) T[k] = st.d[k * st.np + h];
+            sum = st.d[P::NX * st.np + h];
+        }
+        const int w0 = (int)c * chunk, w1 = w0 + chunk < p.W ? w0 + chunk : p.W;
+        pair_windows<SYS>(p, a, odd, T, sum, w0, w1);
+        if (w1 < p.W) {
+#pragma unroll
+            for (int k = 0; k < P::NX; ++k) st.d[k * st.np + h] = T[k];
+            st.d[P::NX * st.np + h] = sum;
+        } else if (!odd && (h >> 1) < p.n_points) {
+            out[q] = sum / p.tMax;
+        }
+    });
+}
+
 LleArgs make_lle_args(const chaos_options& o, double tMax, double NT, int nPts, double h, double eps,
                       const double* ic, int nx, const double* ranges, const int* idx,
                       double transientTime, const double* values, int na)
@@ -107,6 +233,39 @@ static double* lane_state(CallCtx& ctx, int nd, long long groups)
     return static_cast<double*>(ctx.scratch(CallCtx::SCRATCH_STATE, (size_t)nd * groups * 64 * sizeof(double)));
 }
 
+// Transient on one lane per point, then the windows on lane pairs.
+static void launch_lle_split(CallCtx& ctx, int system, const LleArgs& p, int block, double* d_out)
+{
+    const long long n = p.n_points, pairs = (2 * n + 63) / 64;
+    const int turn = rotate_waves(ROTATE_LLE, pairs, device_simds(ctx), (long long)p.W * p.NTp);
+    dispatch_system(system, [&](auto tag) {
+        constexpr int S = decltype(tag)::value;
+        constexpr int NX = System<S>::NX;
+        // the transient's states, then the rotating windows' lane state
+        double* mem = lane_state(ctx, NX + (turn ? NX + 1 : 0), pairs);
+        double* xs = nullptr;
+        const long long xn = pairs * 64;
+        if (p.S > 0) {
+            xs = mem;
+            hipLaunchKernelGGL(lle_transient_kernel<S>, dim3(ceil_div(n, block)), dim3(block), 0, ctx.stream(), p, xs,
+                               xn);
+            ctx.add_launch();
+        }
+        if (turn) {
+            const int chunk = (int)(rotate_chunk_ticks((long long)p.W * p.NTp, p.NTp) / p.NTp);
+            const RotateCtl ctl = make_rotate_ctl(ctx, pairs, (p.W + chunk - 1) / chunk);
+            const LaneStore st{mem + NX * xn, nullptr, xn};
+            hipLaunchKernelGGL(lle_pair_rotate_kernel<S>, dim3(rotate_grid(ctx, turn)), dim3(256), 0, ctx.stream(), p,
+                               ctl, chunk, xs, xn, st, d_out);
+        } else {
+            hipLaunchKernelGGL(lle_pair_kernel<S>, dim3(ceil_div(2 * n, block)), dim3(block), 0, ctx.stream(), p, xs,
+                               xn, d_out);
+        }
+    });
+    CHAOS_HIP(hipGetLastError());
+    ctx.add_launch();
+}
+
 void launch_lle_rows(CallCtx& ctx, int system, LleArgs p, long long row0, long long rows, double* d_out)
 {
     p.row0 = row0;
@@ -114,7 +273,11 @@ void launch_lle_rows(CallCtx& ctx, int system, LleArgs p, long long row0, long l
     const int block = ctx.opt().block > 0 ? ctx.opt().block : 256;
     CHAOS_REQUIRE(block % 64 == 0 && block <= 256, "block must be a multiple of 64 and <= 256");
     const long long groups = (p.n_points + 63) / 64, simds = device_simds(ctx);
-    const long long total = (long long)p.S + (long long)p.W * p.NTp;
+    const long long windows = (long long)p.W * p.NTp, total = (long long)p.S + windows;
+    if (lle_split(groups, simds, windows)) {
+        launch_lle_split(ctx, system, p, block, d_out);
+        return;
+    }
     const int turn = rotate_waves(ROTATE_LLE, groups, simds, total);
     dispatch_system(system, [&](auto tag) {
         constexpr int S = decltype(tag)::value;

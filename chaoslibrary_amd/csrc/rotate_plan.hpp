@@ -58,4 +58,17 @@ inline long long rotate_chunk_ticks(long long ticks, long long unit)
     return (c + unit - 1) / unit * unit;
 }
 
+// Exponent maps: whether the windows run with the base and the perturbed
+// trajectory of a point on two neighbouring lanes instead of one after the
+// other on the same lane.  That halves each wavefront's instructions and
+// doubles the wavefronts: a gain while SIMDs are without one (17^2 points, 2100
+// window ticks: 384 -> 251 us; Rossler with half its 80,000 ticks in windows
+// 128^2 9.2 -> 6.4 ms, 200^2 9.3 -> 7.6, 230^2 (0.81 wavefronts per SIMD) 9.2 ->
+// 8.8), none when they are full (256^2: 9.7 -> 10.0, so the line is at 0.9).
+// window_ticks = W * NTp: below 200 the second launch costs what it saves.
+inline bool lle_split(long long groups, long long simds, long long window_ticks)
+{
+    return simds > 0 && 10 * groups <= 9 * simds && window_ticks >= 200;
+}
+
 }  // namespace chaos

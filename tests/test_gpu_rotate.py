@@ -1,6 +1,7 @@
 """Grids between one and eight wavefronts per SIMD: the wavefronts take turns
-on the SIMDs, with the lane state parked between chunks of ticks.  Results do
-not depend on it: compared with the oracle on sampled rows, with the same map
+on the SIMDs, with the lane state parked between chunks of ticks, and small
+exponent maps run a point's two trajectories on two lanes.  Results do not
+depend on either: compared with the oracle on sampled rows, with the same map
 computed in ranges too small to rotate, and with the job server's."""
 import numpy as np
 import pytest
@@ -28,6 +29,20 @@ def _lle_rows(chaos, oracle, system, s, n, CT, TT, sem, rows, eps=1e-7):
 @pytest.mark.parametrize("sem", [0, 1])
 def test_rotating_exponent_map_matches_oracle(chaos, oracle, sem):
     _lle_rows(chaos, oracle, "rossler_rk4", ROS, 260, 210.0, 40.0, sem, [0, 131, 259])
+
+
+# 2 * 200^2 trajectories on 1250 wavefronts: the windows rotate
+def test_rotating_lane_pairs_match_oracle(chaos, oracle):
+    _lle_rows(chaos, oracle, "chameleon", CHAM, 200, 250.0, 5.0, 0, [0, 100, 199])
+
+
+@pytest.mark.parametrize("n", [1, 2, 5, 6, 17])
+@pytest.mark.parametrize("CT,TT", [(2.0, 0.0), (2.49, 3.0), (7.0, 1.37)])
+def test_lane_pairs_match_oracle_at_small_sizes(chaos, oracle, n, CT, TT):
+    for system, s in (("rossler_rk4", ROS), ("basins_2", dict(values=[0.5, 0.1], ic=[0.3, -0.2],
+                                                              ranges=[0.4, 0.6, 0.05, 0.2], idx=[0, 1]))):
+        for sem in (0, 1):
+            _lle_rows(chaos, oracle, system, s, n, CT, TT, sem, [0, n - 1])
 
 
 @pytest.mark.parametrize("system,s,sem", [("lorenz_rk4", LOR, 1), ("chameleon", CHAM, 0), ("lorenz_rk4", LOR, 0)])
