@@ -37,19 +37,22 @@ constexpr unsigned kRotatePolls = 1u << 27;
 // reports the call as failed.  The state crosses the XCDs' L2 caches between
 // chunks: parked and released at agent scope, acquired before it is loaded.
 //
-// The ticket is read from the first active lane, so the lanes must come to it
-// together: every trip ends in a wave barrier, which keeps lanes that skip a
-// divergent tail of the body (or of the hand-over) from taking the back edge on
-// their own.
+// Lane 0 takes the ticket for the wave, so the lanes must come to it together:
+// every trip ends in a wave barrier, which keeps lanes that skip a divergent
+// tail of the body (or of the hand-over) from taking the back edge on their own.
 template <class Body>
 __device__ __forceinline__ void rotate(const RotateCtl& ctl, Body&& body)
 {
     const int lane = threadIdx.x & 63;
     const unsigned total = ctl.groups * ctl.chunks;
     for (unsigned trip = 0; trip <= total; ++trip) {
-        // one ticket a wave: its 64 lanes add 1 each (one atomic of 64), the
-        // first lane gets the sum before them
-        const unsigned t = __builtin_amdgcn_readfirstlane(atomicAdd(ctl.head, 1u)) >> 6;
+        // one ticket a wave: lane 0 takes it (the lanes are together here).  An
+        // add by all 64 lanes would hand out 64 numbers, which are one atomic
+        // only where the compiler happens to combine them
+        unsigned t = 0;
+        if (lane == 0) t = __hip_atomic_fetch_add(ctl.head, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_wave_barrier();
+        t = __builtin_amdgcn_readfirstlane(t);
         if (t >= total) break;
         const unsigned c = t / ctl.groups, g = t - c * ctl.groups;
         if (c > 0) {
