@@ -132,7 +132,9 @@ void engine_sweep_kernel(const JobDev* __restrict__ jobs, const Tile* __restrict
     drain_family(tiles, ctl, FAM, [&](const Tile& T, int lane) {
         const JobDev& J = jobs[T.slot];
         if (!tile_ok(J, T, FAM, &ctl->err)) return;
-        sweep_group_ticks<SYS, KIND, WV>(J.sw, J.st, J.cursors, J.total, T.group, lane, T.g0, T.g1);
+        sweep_group_ticks<SYS, KIND, WV>(
+            J.sw, [&] { return SweepPark{J.st, J.cursors, J.total}; }, [&] { return (long long)T.group; }, lane, T.g0,
+            T.g1);
     });
 }
 

@@ -237,7 +237,8 @@ struct SweepProg {
     static constexpr bool BIF = stores_peaks(KIND);
     // peak times: the intervals of the bifurcation lists and of the
     // reference basins features; the other kinds use peak values only
-    WavePeakDetector<KIND == KIND_BIF || KIND == KIND_BASINS_REF> det;
+    static constexpr bool DET_TIMES = KIND == KIND_BIF || KIND == KIND_BASINS_REF;
+    WavePeakDetector<DET_TIMES> det;
     int cnt, prev_t;
     unsigned long long alive;  // wave mask of the lanes still integrating
     bool fixed;
@@ -423,20 +424,29 @@ struct SweepProg {
     }
 
     // Recorded samples t, t + 1, ... inside the record (2 <= t, t + 1 < end),
-    // two to a trip; returns the first sample not taken.  A peak or a plateau
-    // can only begin where the samples stop rising (up & c2), and the rest of
-    // the detector matters only while a plateau is open or an index is skipped
-    // (busy): one mask says that a pair needs nothing but its steps, and the
-    // divergence band joins it.  The mask is branched on after the second
-    // sample's steps, which do not depend on it (a compare that is branched on
-    // at once stalls a lone wavefront for the time of about six instructions);
-    // the pairs that need no work run in a loop of their own, so that the state
-    // of the detector and of the peak store is not merged back on every trip.
-    // A lone wavefront issues one instruction per 6 clocks whatever its kind,
-    // so fewer scalar instructions and branches a sample count there: the
-    // Rossler diagram of 1000 points 28.9 -> 21.1 ms, BASINS basins of 200^2
-    // 73.5 -> 57.9 ms.  Full grids are bound by FP64 issue and stay (Lorenz
-    // peak map 1024^2 91.4 -> 91.6 ms, basins 1024^2 96.4 -> 95.3 ms).
+    // two to a trip; returns the first sample not taken.
+    //
+    // A peak needs a rising sample followed by a fall (up & c2 & ~tiny) and
+    // nothing more unless a plateau is open or begins or an index is skipped;
+    // such a peak only joins its lane's pending slot (a masked move).  The slots
+    // are emptied together -- one append, or one masked update of the sums --
+    // when a lane with a full slot peaks again: lanes peak every 30 to 600
+    // samples but some lane of the 64 nearly every sample, so that work runs
+    // once for tens of peaks.  A pair with anything else to it -- a plateau, a
+    // value outside the divergence band, a second peak -- goes sample by sample
+    // (settle).  Its mask is branched on after the second sample's steps, which
+    // do not depend on it (a compare that is branched on at once stalls a lone
+    // wavefront for the time of about six instructions), and the pairs that do
+    // not need it run in a loop of their own, so that the state of the detector
+    // and of the peak store is not merged back on every trip.
+    //
+    // A lone wavefront pays an issue slot per instruction of any kind, so fewer
+    // scalar instructions and branches a sample count there: the Rossler diagram
+    // of 1000 points 28.9 -> 21.1 ms with the pairs, BASINS basins of 200^2
+    // 73.5 -> 57.9 ms.  The pending slots: Lorenz peak map 88.8 -> 86.2 ms at
+    // 1024^2 points and (sweep alone) 8.1 -> 6.9 ms at 200^2, basins 93.1 ->
+    // 91.6 ms at 1024^2; full grids are bound by FP64 issue.  Chameleon's long
+    // steps leave them nothing to gain (31.2 -> 31.3 ms at 300^2).
     template <int WVT, bool PRE1>
     __device__ __forceinline__ int body(const SweepArgs& A, int wv, WaveCursor& cur, int wave, int t, int end)
     {
@@ -448,9 +458,12 @@ struct SweepProg {
         unsigned long long busy = det.m.busy();
         double p = det.p;
         unsigned long long up = det.m.up;
+        unsigned long long pend = 0ull;  // lanes with a full slot (value pend_v, time pend_t)
+        double pend_v = 0.0;
+        int pend_t = 0;
         while (t + 1 < end) {
             double v0, v1;
-            unsigned long long c0, c1, y0, y1, o0, o1, event;
+            unsigned long long c0, c1, y0, y1, o0, o1, other;
             do {
                 det.p = p;  // the history before the pair
                 det.m.up = up;
@@ -465,23 +478,57 @@ struct SweepProg {
                 c1 = wave_mask(d1 <= 0.0);
                 y1 = wave_mask(fabs(d1) <= 1e-13);
                 o1 = wave_mask(!(fabs(v1) < A.L));
-                event = (c0 & up) | (c1 & ~(c0 | y0)) | ((o0 | o1) & alive) | busy;
+                // rising samples followed by one that does not rise
+                const unsigned long long f0 = up & c0, f1 = c1 & ~(c0 | y0);
+                other = ((o0 | o1) & alive) | busy;
                 advance();
                 pin_state();
                 t += 2;
+                if (f0 | f1 | other) {
+                    const unsigned long long e0 = f0 & ~y0 & alive, e1 = f1 & ~y1 & alive;
+                    other |= (f0 & y0) | (f1 & y1) | ((e0 | e1) & pend);
+                    if (other) break;
+                    // the peaks are the samples t - 3 and t - 2 now
+                    masked_move(pend_v, p, e0, v0, e1);
+                    if (DET_TIMES) masked_move(pend_t, t - 3, e0, t - 2, e1);
+                    pend |= e0 | e1;
+                }
                 p = v1;
                 up = ~(c1 | y1);
-            } while (event == 0ull && t + 1 < end);
-            if (event) {
+            } while (t + 1 < end);
+            if (other) {
+                if (pend) on_peaks(A, cur, wave, pend, pend_v, pend_t);
+                pend = 0ull;
                 settle(A, cur, wave, t - 2, v0, c0, y0, o0);
                 settle(A, cur, wave, t - 1, v1, c1, y1, o1);
                 busy = det.m.busy();
+                p = det.p;
+                up = det.m.up;
             }
         }
+        if (pend) on_peaks(A, cur, wave, pend, pend_v, pend_t);
         det.p = p;
         det.m.up = up;
         check<WVT>(A, wv);  // the last pair's second step
         return t;
+    }
+
+    // to = a on lanes m, b on lanes n (disjoint).  All 64 lanes are active.
+    __device__ __forceinline__ static void masked_move(double& to, double a, unsigned long long m, double b,
+                                                       unsigned long long n)
+    {
+        asm volatile("s_mov_b64 exec, %3\n\tv_mov_b64 %0, %1\n\ts_mov_b64 exec, %4\n\tv_mov_b64 %0, %2\n\t"
+                     "s_mov_b64 exec, -1"
+                     : "+v"(to)
+                     : "v"(a), "v"(b), "s"(m), "s"(n));
+    }
+    __device__ __forceinline__ static void masked_move(int& to, int a, unsigned long long m, int b,
+                                                       unsigned long long n)
+    {
+        asm volatile("s_mov_b64 exec, %3\n\tv_mov_b32 %0, %1\n\ts_mov_b64 exec, %4\n\tv_mov_b32 %0, %2\n\t"
+                     "s_mov_b64 exec, -1"
+                     : "+v"(to)
+                     : "s"(a), "s"(b), "s"(m), "s"(n));
     }
 
     // Keeps the steps before this point ahead of the branch that follows.
@@ -648,38 +695,52 @@ struct SweepProg {
     }
 };
 
-// Ticks [g0, g1) of one 64-point group of a sweep whose lane state is parked in
-// st (and, for the kinds that store peaks, its peak-store cursor in cursors)
-// between calls; writes the outputs when g1 is the last tick.  All 64 lanes of
-// the wave call it.
-template <int SYS, int KIND, int WV>
-__device__ __forceinline__ void sweep_group_ticks(const SweepArgs& A, const LaneStore& st, WaveCursor* cursors,
-                                                  long long total, long long group, int lane, long long g0,
-                                                  long long g1)
+// Where a sweep group's state is parked between calls.
+struct SweepPark {
+    LaneStore st;
+    WaveCursor* cursors;  // per group, for the kinds that store peaks
+    long long total;      // ticks of the whole run
+};
+
+// Ticks [g0, g1) of one 64-point group of a sweep whose lane state is parked
+// between calls; writes the outputs when g1 is the last tick.  park() gives the
+// SweepPark and is called anew after the ticks, so that it need not stay in
+// registers across them.  All 64 lanes of the wave call it.
+template <int SYS, int KIND, int WV, class Park, class G>
+__device__ __forceinline__ void sweep_group_ticks(const SweepArgs& A, const Park& park, const G& group_of, int lane,
+                                                  long long g0, long long g1)
 {
-    const long long q = group * 64 + lane;
-    const bool in_range = q < A.n_points;
-    const long long pq = A.p0 + (in_range ? q : 0);
     SweepProg<SYS, KIND> L;
     WaveCursor cur{A.pool.nchunks, kChunk};
-    if (g0 == 0) {
-        L.init(A, pq, in_range);
-    } else {
-        L.params(A, pq);
-        L.load(st, q);
-        if (stores_peaks(KIND)) {
-            const WaveCursor c = cursors[group];
-            cur.chunk = __builtin_amdgcn_readfirstlane(c.chunk);
-            cur.fill = __builtin_amdgcn_readfirstlane(c.fill);
+    const long long group = group_of();
+    {
+        const SweepPark P = park();
+        const long long q = group * 64 + lane;
+        const bool in_range = q < A.n_points;
+        const long long pq = A.p0 + (in_range ? q : 0);
+        if (g0 == 0) {
+            L.init(A, pq, in_range);
+        } else {
+            L.params(A, pq);
+            L.load(P.st, q);
+            if (stores_peaks(KIND)) {
+                const WaveCursor c = P.cursors[group];
+                cur.chunk = __builtin_amdgcn_readfirstlane(c.chunk);
+                cur.fill = __builtin_amdgcn_readfirstlane(c.fill);
+            }
         }
     }
+    const bool last = g1 == park().total;
     L.template ticks<WV>(A, WV, cur, (int)group, g0, g1);
-    if (g1 == total) {
+    const long long after = group_of();
+    const long long q = after * 64 + lane;
+    if (last) {
         if (stores_peaks(KIND)) close_chunk(A.pool, cur);
-        if (in_range) L.finish(A, q);
+        if (q < A.n_points) L.finish(A, q);
     } else {
-        L.store(st, q);
-        if (stores_peaks(KIND) && lane == 0) cursors[group] = cur;
+        const SweepPark P = park();
+        L.store(P.st, q);
+        if (stores_peaks(KIND) && lane == 0) P.cursors[after] = cur;
     }
 }
 

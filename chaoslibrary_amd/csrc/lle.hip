@@ -42,25 +42,33 @@ void lle_map_kernel(const LleArgs p, double* __restrict__ out)
 // ticks of 64-point groups, the lane state parked in st between them.  Rossler
 // map of 300^2 points (1.4 wavefronts per SIMD, 240,100 ticks): 41.0 -> 29.3 ms.
 template <int SYS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void lle_rotate_kernel(const LleArgs p, const RotateCtl ctl, long long chunk, const LaneStore st,
                        double* __restrict__ out)
 {
     using P = LleProg<SYS>;
-    const long long total = P::total(p);
+    struct Kept {
+        LaneStore st;
+        double* out;
+        long long chunk;
+    };
+    const InVgprs<Kept> kept(Kept{st, out, chunk});
     rotate(ctl, [&](unsigned g, unsigned c, int lane) {
         const long long q = (long long)g * 64 + lane;
         const long long qq = q < p.n_points ? q : 0;
         const int i = (int)(qq % p.nPts);
         const int j = (int)(p.row0 + qq / p.nPts);
+        const Kept k = kept.get();
         P L;
         L.params(p, i, j);
         if (c == 0) L.init(p);
-        else L.load(st, q);
-        const long long g0 = (long long)c * chunk, g1 = g0 + chunk < total ? g0 + chunk : total;
+        else L.load(k.st, q);
+        const long long total = P::total(p), g0 = (long long)c * k.chunk;
+        const long long g1 = g0 + k.chunk < total ? g0 + k.chunk : total;
         L.ticks(p, (long long)j * p.nPts + i, g0, g1);
-        if (g1 < total) L.store(st, q);
-        else if (q < p.n_points) out[q] = L.result(p);
+        const Kept after = kept.get();
+        if (g1 < total) L.store(after.st, q);
+        else if (q < p.n_points) after.out[q] = L.result(p);
     });
 }
 

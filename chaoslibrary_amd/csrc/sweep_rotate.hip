@@ -12,14 +12,18 @@
 namespace chaos {
 
 template <int SYS, int WV, int KIND>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void sweep_rotate_kernel(const SweepArgs A, const RotateCtl ctl, long long chunk, const LaneStore st,
                          WaveCursor* __restrict__ cursors)
 {
     const long long total = SweepProg<SYS, KIND>::total(A);
+    const InVgprs<SweepPark> park(SweepPark{st, cursors, total});
+    const InVgprs<long long> len(chunk);
     rotate(ctl, [&](unsigned g, unsigned c, int lane) {
-        const long long g0 = (long long)c * chunk, g1 = g0 + chunk < total ? g0 + chunk : total;
-        sweep_group_ticks<SYS, KIND, WV>(A, st, cursors, total, g, lane, g0, g1);
+        const InVgprs<long long> group((long long)g);
+        const long long n = len.get(), g0 = (long long)c * n, left = park.get().total - g0;
+        sweep_group_ticks<SYS, KIND, WV>(
+            A, [&] { return park.get(); }, [&] { return group.get(); }, lane, g0, g0 + (n < left ? n : left));
     });
 }
 
