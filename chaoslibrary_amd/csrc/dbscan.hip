@@ -215,10 +215,15 @@ __device__ __forceinline__ int lookup(const GridDev& G, unsigned long long key)
     return -1;
 }
 
+__device__ __forceinline__ int uf_load(const int* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
 // Slot of `key`, inserting it if absent.  A non-empty slot never changes, so
 // a plain load that sees a key is final; an empty one is claimed by
 // compare-and-swap.  A table more than half full is flagged (the host redoes
-// the clustering with the larger table); a full one returns -1.
+// the clustering with the larger table) and a search in it ends after eight
+// probes: nothing of the pass is used any more, and filled up, every insertion
+// would walk all of it (300,000 scattered points, a cell each: 10.9 s, 3.3 ms
+// so).
 __device__ __forceinline__ int hash_insert(const GridDev& G, unsigned long long key)
 {
     unsigned long long h = mix64(key) & G.hmask;
@@ -234,6 +239,7 @@ __device__ __forceinline__ int hash_insert(const GridDev& G, unsigned long long 
             if (prev == key) return (int)h;
         }
         h = (h + 1) & G.hmask;
+        if ((probe & 7) == 7 && (uf_load(&G.ctl->flags) & DB_FULL)) return -1;
     }
     atomicOr(&G.ctl->flags, DB_FULL);
     return -1;
@@ -284,8 +290,6 @@ __device__ __forceinline__ int box_relation(const GridDev& G, long long p, int s
     if (sqrt(f2) <= G.eps) return 2;
     return 1;
 }
-
-__device__ __forceinline__ int uf_load(const int* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 __device__ __forceinline__ int uf_find(const GridDev& G, int x)
 {
@@ -350,11 +354,31 @@ __device__ __forceinline__ unsigned long long lanes_below() { return (1ull << __
 // Lanes left pending afterwards (many distinct keys) update on their own.
 constexpr int kAggGroups = 4;
 
-// Per-block chunks of the aggregated kernels: 256 threads x kPer points,
-// consecutive point indices per pass, and an LDS table of kLds cells.
-constexpr int kPer = 8;
-constexpr int kChunkPts = 256 * kPer;
+// Per-block chunks of the aggregated kernels: 256 threads x PER points,
+// consecutive point indices per pass, and an LDS table of kLds cells.  A long
+// chunk saves global atomics on the cells that many points share; a short one
+// fills the chip, and at PER = 1 the table holds every cell its 256 points can
+// lie in.  Whole clustering, 8 points a thread -> the rule below: 8,000 points
+// 0.24 -> 0.14 ms, 160,000 0.71 -> 0.65 ms, 300,000 1.07 -> 1.02 ms, the same
+// from 524,288 on.
+constexpr int kMaxPer = 8;
 constexpr int kLds = 512;
+// Probes of the LDS table before a key goes to the global one.  A chunk of
+// scattered points has more cells than the table has entries, and every point
+// past the 512th would walk all of it.
+constexpr int kLdsProbes = 16;
+
+// Points per thread: the most that leaves a block for each of 256 CUs.
+static int chunk_per(long long n)
+{
+    int per = kMaxPer;
+    while (per > 1 && n < 256LL * per * 256) per >>= 1;
+    return per;
+}
+
+// Items of a wavefront-per-item kernel: none once the cell table has overflowed,
+// when nothing of the pass is used.
+__device__ __forceinline__ int items(const GridDev& G, int count) { return G.ctl->flags & DB_FULL ? 0 : count; }
 
 // Grid of the wavefront-per-item kernels (blocks of 256): 8192 waves, a full
 // complement for 256 CUs; the waves stride over the device-side item count.
@@ -483,11 +507,12 @@ __global__ void setup_kernel(const GridDev G, double cell_lim)
     }
 }
 
-// Slot of `key` in the block's LDS table, claiming it if absent; -1 if full.
+// Slot of `key` in the block's LDS table, claiming it if absent; -1 if there is
+// no room near its place (a key once refused is refused again: entries stay).
 __device__ __forceinline__ int lds_claim(unsigned long long* s_key, unsigned long long key)
 {
     int h = (int)(mix64(key) & (kLds - 1));
-    for (int probe = 0; probe < kLds; ++probe) {
+    for (int probe = 0; probe < kLdsProbes; ++probe) {
         const unsigned long long k = s_key[h];
         if (k == key) return h;
         if (k == kEmpty) {
@@ -502,6 +527,7 @@ __device__ __forceinline__ int lds_claim(unsigned long long* s_key, unsigned lon
 // Cells of the included points: count, smallest member index and member box
 // per cell, aggregated over the wavefront, then over the block's chunk in
 // LDS, then added to the global table once per cell and block.
+template <int PER>
 __global__ __launch_bounds__(256) void insert_kernel(const GridDev G)
 {
     __shared__ unsigned long long s_key[kLds];
@@ -521,9 +547,9 @@ __global__ __launch_bounds__(256) void insert_kernel(const GridDev G)
     }
     __syncthreads();
     // per point: LDS entry (>= 0), a global slot s encoded as -2 - s, or -1
-    int loc[kPer];
-    const long long base = (long long)blockIdx.x * kChunkPts;
-    for (int k = 0; k < kPer; ++k) {
+    int loc[PER];
+    const long long base = (long long)blockIdx.x * (256 * PER);
+    for (int k = 0; k < PER; ++k) {
         const long long p = base + (long long)k * 256 + tid;
         const bool valid = p < G.n && included(G, p);
         unsigned long long key = kEmpty, e[3] = {0ull, 0ull, 0ull};
@@ -603,7 +629,7 @@ __global__ __launch_bounds__(256) void insert_kernel(const GridDev G)
         s_slot[i] = slot;
     }
     __syncthreads();
-    for (int k = 0; k < kPer; ++k) {
+    for (int k = 0; k < PER; ++k) {
         const long long p = base + (long long)k * 256 + tid;
         if (p >= G.n) break;
         const int l = loc[k];
@@ -611,11 +637,11 @@ __global__ __launch_bounds__(256) void insert_kernel(const GridDev G)
     }
 }
 
-// Slot of an int key in an LDS table of kLds entries (-1 = empty).
+// The same for an int key (-1 = empty).
 __device__ __forceinline__ int lds_claim_int(int* s_key, int key)
 {
     int h = (int)(mix64((unsigned long long)key) & (kLds - 1));
-    for (int probe = 0; probe < kLds; ++probe) {
+    for (int probe = 0; probe < kLdsProbes; ++probe) {
         const int k = s_key[h];
         if (k == key) return h;
         if (k == -1) {
@@ -632,6 +658,7 @@ __device__ __forceinline__ int lds_claim_int(int* s_key, int key)
 // dense part of the core test: a cell holding >= minPts points is all-core
 // (its diagonal is below eps) and its members link straight to its smallest
 // member; points of sparser cells go to the candidate list.
+template <int PER>
 __global__ __launch_bounds__(256) void place_kernel(const GridDev G, int minPts)
 {
     __shared__ int s_slot[kLds];
@@ -643,9 +670,9 @@ __global__ __launch_bounds__(256) void place_kernel(const GridDev G, int minPts)
         s_cnt[i] = 0;
     }
     __syncthreads();
-    int loc[kPer], rank[kPer], sl[kPer];  // loc: LDS entry, -2 = placed directly, -1 = none
-    const long long base = (long long)blockIdx.x * kChunkPts;
-    for (int k = 0; k < kPer; ++k) {
+    int loc[PER], rank[PER], sl[PER];  // loc: LDS entry, -2 = placed directly, -1 = none
+    const long long base = (long long)blockIdx.x * (256 * PER);
+    for (int k = 0; k < PER; ++k) {
         const long long p = base + (long long)k * 256 + tid;
         const int s = p < G.n ? G.pslot[p] : -1;
         sl[k] = s;
@@ -690,7 +717,7 @@ __global__ __launch_bounds__(256) void place_kernel(const GridDev G, int minPts)
         s_base[i] = s >= 0 ? G.hstart[s] + atomicAdd(&G.hcur[s], s_cnt[i]) : 0;
     }
     __syncthreads();
-    for (int k = 0; k < kPer; ++k) {
+    for (int k = 0; k < PER; ++k) {
         const long long p = base + (long long)k * 256 + tid;
         const int l = loc[k];
         if (l >= 0) G.cellpts[s_base[l] + rank[k]] = (int)p;
@@ -813,7 +840,7 @@ __global__ __launch_bounds__(256) void core_sparse_kernel(const GridDev G, int m
     const int lane = __lane_id();
     const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const long long nw = ((long long)gridDim.x * blockDim.x) >> 6;
-    const int nc = G.ctl->ncand;
+    const int nc = items(G, G.ctl->ncand);
     for (long long i = wave; i < nc; i += nw) {
         const int p = G.cand[i];
         int sl[2], rl[2];
@@ -924,7 +951,7 @@ __global__ __launch_bounds__(256) void border_sparse_kernel(const GridDev G)
     const int lane = __lane_id();
     const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const long long nw = ((long long)gridDim.x * blockDim.x) >> 6;
-    const int nc = G.ctl->ncand;
+    const int nc = items(G, G.ctl->ncand);
     for (long long i = wave; i < nc; i += nw) {
         const int p = G.cand[i];
         if (G.parent[p] >= 0) continue;  // core (uniform over the wavefront)
@@ -1066,7 +1093,7 @@ __global__ __launch_bounds__(256) void link_pairs_kernel(const GridDev G, int ri
     const int lane = __lane_id();
     const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const long long nw = ((long long)gridDim.x * blockDim.x) >> 6;
-    const int nc = G.ctl->ncore_cells;
+    const int nc = items(G, G.ctl->ncore_cells);
     const int noff = G.dim == 3 ? 125 : 25;
     for (long long i = wave; i < nc; i += nw) {
         const int a = G.cells[i];
@@ -1245,10 +1272,19 @@ static DbCtl run_pipeline(CallCtx& ctx, GridDev& G, const DbscanParams& prm, int
     hipLaunchKernelGGL(init_kernel, dim3(gi), dim3(T), 0, st, G, box, 1);
     if (!box) hipLaunchKernelGGL(bbox_kernel, dim3(std::min<unsigned>(gn, 1024u)), dim3(T), 0, st, G);
     hipLaunchKernelGGL(setup_kernel, dim3(1), dim3(64), 0, st, G, cell_lim);
-    const unsigned gc = ceil_div(n, kChunkPts);
-    hipLaunchKernelGGL(insert_kernel, dim3(gc), dim3(T), 0, st, G);
+    const int per = chunk_per(n);
+    const unsigned gc = ceil_div(n, 256 * per);
+    hipLaunchKernelGGL(per == 8   ? insert_kernel<8>
+                       : per == 4 ? insert_kernel<4>
+                       : per == 2 ? insert_kernel<2>
+                                  : insert_kernel<1>,
+                       dim3(gc), dim3(T), 0, st, G);
     scan_i32(st, reinterpret_cast<const int*>(G.hcount), G.hstart, G.H, G.scan_tmp);
-    hipLaunchKernelGGL(place_kernel, dim3(gc), dim3(T), 0, st, G, prm.minPts);
+    hipLaunchKernelGGL(per == 8   ? place_kernel<8>
+                       : per == 4 ? place_kernel<4>
+                       : per == 2 ? place_kernel<2>
+                                  : place_kernel<1>,
+                       dim3(gc), dim3(T), 0, st, G, prm.minPts);
     hipLaunchKernelGGL(cell_init_kernel, dim3(gh), dim3(T), 0, st, G, prm.minPts);
     hipLaunchKernelGGL(core_sparse_kernel, dim3(kWaveBlocks), dim3(T), 0, st, G, prm.minPts);
     hipLaunchKernelGGL(core_piece_kernel, dim3(kWaveBlocks), dim3(T), 0, st, G, prm.minPts);

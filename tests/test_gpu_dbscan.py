@@ -159,3 +159,20 @@ def test_dbscan_split_core_tests_match_bruteforce(chaos, oracle, capfd, monkeypa
     pieces, cap = map(int, re.search(r"(\d+) split pieces of (\d+)", line).groups())
     assert pieces > 0 and pieces + 5 > cap  # the list was used and filled
     assert 0 < (cnt >= 300).sum() < 300
+
+
+# Pairs of points on a lattice, a cell or two to each pair: labels known without
+# a search.  Sizes around the chunks' ends and around the points per thread;
+# from 131,073 pairs on the first cell table overflows.
+@pytest.mark.parametrize("n", [1, 255, 257, 131071, 131072, 262145, 300001, 524288, 600001])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_gpu_lattice_pairs(chaos, n, dim):
+    eps = 0.25
+    p = np.arange(n)
+    i = p // 2
+    m = 700
+    pts = np.stack([(i % m) * 1.0 + (p % 2) * 0.125, (i // m) * 1.0, (i % 7) * 2.0][:dim], axis=1)
+    print(f"lattice pairs n={n} dim={dim}", flush=True)
+    labels, k = chaos.dbscan(pts, eps, 1)
+    assert k == (n + 1) // 2
+    assert np.array_equal(labels, i + 1)
