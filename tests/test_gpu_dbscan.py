@@ -176,3 +176,28 @@ def test_gpu_lattice_pairs(chaos, n, dim):
     labels, k = chaos.dbscan(pts, eps, 1)
     assert k == (n + 1) // 2
     assert np.array_equal(labels, i + 1)
+
+
+# A spread crowd of n points in one cell, a tight group and single points that
+# only the crowd's outermost members reach, and (ring) points around it at
+# distances near eps: links and border searches that the crowd's first 512
+# members do not decide, and whose rest is walked in pieces of 4096.
+@pytest.mark.parametrize("n", [512, 513, 4608, 4609, 20000])
+@pytest.mark.parametrize("min_pts", [20, 4])
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("ring", [0, 600])
+def test_gpu_crowded_cell_walked_in_pieces(chaos, oracle, n, min_pts, dim, ring):
+    rng = np.random.default_rng(n + min_pts)
+    eps = 0.5
+    crowd = rng.uniform(0.0, 0.28, size=(n, dim))
+    around = rng.normal(size=(ring, dim))
+    around *= (rng.uniform(0.3, 0.75, size=ring) / np.linalg.norm(around, axis=1))[:, None]
+    group = np.array([0.776] + [0.1] * (dim - 1)) + rng.uniform(0.0, 0.004, size=(40, dim))
+    singles = rng.uniform(0.0, 0.28, size=(8 if min_pts == 20 else 2, dim))
+    singles[:, 0] = -0.496 - rng.uniform(0.0, 0.004, size=len(singles))
+    pts = np.concatenate([crowd, 0.14 + around, group, singles])
+    pts = pts[rng.permutation(len(pts))]
+    print(f"crowd n={n} min_pts={min_pts} dim={dim} ring={ring}", flush=True)
+    labels, k = chaos.dbscan(pts, eps, min_pts)
+    want = oracle.dbscan_bruteforce(pts, eps, min_pts)
+    assert np.array_equal(labels, want)
