@@ -106,6 +106,8 @@ _SIGS = {
                               C.c_int, C.c_char_p]),
     "chaos_dbscan": (C.c_int, [C.POINTER(Options), _D, _D, _D, C.c_longlong, C.c_int, C.c_double, C.c_int,
                                C.c_int, _I, _I, _I]),
+    "chaos_dbscan_rows": (C.c_int, [C.POINTER(Options), _D, C.c_longlong, C.c_int, C.c_double, C.c_int, C.c_int,
+                                    _I, _I, _I]),
 }
 
 
@@ -334,14 +336,12 @@ def dbscan(points, eps, min_pts=20, sign_rule=False, include=None, **kw):
     """chaos_dbscan over points[n, dim] (dim 2 or 3): (labels[n], K)."""
     pts = _f64(points)
     n, dim = pts.shape
-    cols = [np.ascontiguousarray(pts[:, d]) for d in range(dim)]
     inc = None if include is None else _i32(include)
     labels = np.zeros(n, dtype=np.int32)
     k = C.c_int(0)
     o = make_options(**kw)
-    _check(lib.chaos_dbscan(C.byref(o), _dp(cols[0]), _dp(cols[1]), _dp(cols[2]) if dim == 3 else None, n, dim,
-                            float(eps), int(min_pts), 1 if sign_rule else 0, None if inc is None else _ip(inc),
-                            _ip(labels), C.byref(k)))
+    _check(lib.chaos_dbscan_rows(C.byref(o), _dp(pts), n, dim, float(eps), int(min_pts), 1 if sign_rule else 0,
+                                 None if inc is None else _ip(inc), _ip(labels), C.byref(k)))
     return labels, k.value
 
 

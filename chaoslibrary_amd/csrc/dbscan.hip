@@ -1814,16 +1814,54 @@ const double* zscore_moments_device(CallCtx& ctx, const double* const* src, int 
 
 using namespace chaos;
 
-extern "C" int chaos_dbscan(const chaos_options* opt, const double* x, const double* y, const double* z, long long n,
-                            int dim, double eps, int min_pts, int sign_rule, const int* include, int* labels,
-                            int* clusters)
+namespace {
+
+// Points per slab of a row upload (24 MiB of rows in three dimensions).
+constexpr long long kRowSlab = 1LL << 20;
+
+__global__ __launch_bounds__(256) void columns_kernel(const double* __restrict__ rows, long long m, int dim,
+                                                      double* __restrict__ cols, long long n)
 {
-    return guarded("chaos_dbscan", [&] {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= m * dim) return;
+    const long long p = i / dim;
+    cols[(i - p * dim) * n + p] = rows[i];
+}
+
+// Rows of dim coordinates to device columns of n, slab by slab through one
+// buffer (the stream orders a slab's copy behind the kernel that read the last).
+// One copy of what the caller holds and a pass on the device (15 us at a million
+// points) instead of strided column copies on the host (2 ms).
+void upload_rows(CallCtx& ctx, const double* rows, bool dev, long long n, int dim, double* cols)
+{
+    hipStream_t st = ctx.stream();
+    DevBuf<double> slab;
+    if (!dev) slab.alloc((size_t)dim * std::min(n, kRowSlab));
+    for (long long p = 0; p < n; p += kRowSlab) {
+        const long long m = std::min(n - p, kRowSlab);
+        const double* src = rows + p * dim;
+        if (!dev) {
+            CHAOS_HIP(hipMemcpyAsync(slab.get(), src, (size_t)m * dim * 8, hipMemcpyHostToDevice, st));
+            src = slab.get();
+        }
+        hipLaunchKernelGGL(columns_kernel, dim3(ceil_div(m * dim, 256)), dim3(256), 0, st, src, m, dim, cols + p, n);
+        CHAOS_HIP(hipGetLastError());
+        ctx.add_launch(1);
+    }
+    ctx.sync();  // the slab is given back here
+}
+
+// chaos_dbscan on columns x, y, z, or chaos_dbscan_rows on rows.
+int cluster_call(const char* name, const chaos_options* opt, const double* x, const double* y, const double* z,
+                 const double* rows, long long n, int dim, double eps, int min_pts, int sign_rule,
+                 const int* include, int* labels, int* clusters)
+{
+    return guarded(name, [&] {
         chaos_options o = resolve_options(opt);
         CHAOS_REQUIRE(n >= 0 && n < INT_MAX, "n out of range");
         CHAOS_REQUIRE(dim == 2 || dim == 3, "dim must be 2 or 3");
         CHAOS_REQUIRE(sign_rule == 0 || dim == 2, "sign_rule needs dim 2");
-        CHAOS_REQUIRE(x && y && (dim == 2 || z), "coordinate array is NULL");
+        CHAOS_REQUIRE(rows || (x && y && (dim == 2 || z)), "coordinate array is NULL");
         CHAOS_REQUIRE(labels, "labels is NULL");
         CHAOS_REQUIRE(sign_rule || min_pts >= 1, "min_pts must be >= 1");
         if (clusters) *clusters = 0;
@@ -1836,12 +1874,17 @@ extern "C" int chaos_dbscan(const chaos_options* opt, const double* x, const dou
         const double* pts[3] = {x, y, z};
         const int* inc = include;
         int* lab = labels;
-        if (!dev) {
-            d_pts.alloc((size_t)dim * n);
+        if (rows || !dev) d_pts.alloc((size_t)dim * n);
+        if (rows) {
+            upload_rows(ctx, rows, dev, n, dim, d_pts.get());
+            for (int d = 0; d < dim; ++d) pts[d] = d_pts.get() + d * n;
+        } else if (!dev) {
             for (int d = 0; d < dim; ++d) {
                 CHAOS_HIP(hipMemcpyAsync(d_pts.get() + d * n, pts[d], n * 8, hipMemcpyHostToDevice, st));
                 pts[d] = d_pts.get() + d * n;
             }
+        }
+        if (!dev) {
             d_lab.alloc(n);
             lab = d_lab.get();
             if (inc) {
@@ -1859,4 +1902,21 @@ extern "C" int chaos_dbscan(const chaos_options* opt, const double* x, const dou
         if (clusters) *clusters = K;
         ctx.finish();
     });
+}
+
+}  // namespace
+
+extern "C" int chaos_dbscan(const chaos_options* opt, const double* x, const double* y, const double* z, long long n,
+                            int dim, double eps, int min_pts, int sign_rule, const int* include, int* labels,
+                            int* clusters)
+{
+    return cluster_call("chaos_dbscan", opt, x, y, z, nullptr, n, dim, eps, min_pts, sign_rule, include, labels,
+                        clusters);
+}
+
+extern "C" int chaos_dbscan_rows(const chaos_options* opt, const double* points, long long n, int dim, double eps,
+                                 int min_pts, int sign_rule, const int* include, int* labels, int* clusters)
+{
+    return cluster_call("chaos_dbscan_rows", opt, nullptr, nullptr, nullptr, points, n, dim, eps, min_pts, sign_rule,
+                        include, labels, clusters);
 }

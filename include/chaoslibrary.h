@@ -246,6 +246,12 @@ int chaos_dbscan(const chaos_options* opt, const double* x, const double* y,
                  int min_pts, int sign_rule, const int* include, int* labels,
                  int* clusters);
 
+/* chaos_dbscan on points[n][dim] (row-major): one upload of the caller's array,
+ * split into columns on the device. */
+int chaos_dbscan_rows(const chaos_options* opt, const double* points, long long n,
+                      int dim, double eps, int min_pts, int sign_rule,
+                      const int* include, int* labels, int* clusters);
+
 /* No counterpart in the reference.  chaos_dbscan for callers that cannot
  * allocate (code under hipGraph capture, tight serving loops): the same
  * kernels and results, with no hipMalloc, hipFree or other allocation -- the

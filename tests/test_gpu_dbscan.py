@@ -163,8 +163,9 @@ def test_dbscan_split_core_tests_match_bruteforce(chaos, oracle, capfd, monkeypa
 
 # Pairs of points on a lattice, a cell or two to each pair: labels known without
 # a search.  Sizes around the chunks' ends and around the points per thread;
-# from 131,073 pairs on the first cell table overflows.
-@pytest.mark.parametrize("n", [1, 255, 257, 131071, 131072, 262145, 300001, 524288, 600001])
+# from 131,073 pairs on the first cell table overflows; rows go to the device in
+# slabs of 2^20.
+@pytest.mark.parametrize("n", [1, 255, 257, 131071, 131072, 262145, 300001, 524288, 600001, 1048576, 1048577])
 @pytest.mark.parametrize("dim", [2, 3])
 def test_gpu_lattice_pairs(chaos, n, dim):
     eps = 0.25
