@@ -68,7 +68,8 @@ void launch_sweep(CallCtx& ctx, int system, int writableVar, int kind, const Swe
     // A grid of at most one wavefront per CU (a 1-D sweep of 1000 points: 16
     // wavefronts) runs them one per CU in 64-thread blocks, so that a
     // latency-bound wavefront does not share its CU's scalar unit and
-    // instruction issue with three others: 31.9 -> 28.3 ms for that sweep.
+    // instruction issue with three others: 31.9 -> 28.3 ms for that
+    // sweep (20.3 ms with the sample pairs of SweepProg::body).
     // (Grids of a few wavefronts per CU gained nothing and sometimes lost.)
     // The basins epilogue's moments need the 256-thread blocks.
     const bool spread = A.zsum == nullptr &&
