@@ -34,20 +34,61 @@ __global__ void kept_kernel(const int* __restrict__ flags, const int* __restrict
     if (p < n) kept[p] = flags[p] == 1 ? counts[p] : 0;
 }
 
-__global__ void scatter_kernel(const PeakPool pool, unsigned used, const int* __restrict__ flags,
-                               const long long* __restrict__ off, double* __restrict__ vals,
-                               unsigned* __restrict__ times, long long n)
+// Chunk entries to their points' segments, a block to a chunk.  The entries
+// lie in the order the wave found them, so 64 neighbouring ones go to 64
+// points; a chunk holds about four of each point, with consecutive sequence
+// numbers.  They are put in order of (point, sequence) in LDS first, and a store
+// then covers a quarter of the lines (482 M peaks of a 1024^2 map: 5.5 -> 4.0 ms).
+// Loading the 64 segments before the entries are ranked, or several chunks of
+// one wave by one block, was slower (4.7 and 5.6 ms).
+__global__ __launch_bounds__(kChunk) void scatter_kernel(const PeakPool pool, const int* __restrict__ flags,
+                                                         const long long* __restrict__ off,
+                                                         double* __restrict__ vals, unsigned* __restrict__ times,
+                                                         long long n)
 {
-    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const unsigned c = (unsigned)(g / kChunk);
-    const int s = (int)(g % kChunk);
-    if (c >= used || s >= pool.fill()[c]) return;
-    const PeakEntry e = pool.entries[(size_t)c * kChunk + s];
-    const long long p = (long long)pool.owner()[c] * 64 + (e.kl & 63u);
-    if (p >= n || flags[p] != 1) return;
-    const long long pos = off[p] + (e.kl >> 6);
-    if (vals) vals[pos] = e.v;
-    if (times) times[pos] = e.t;
+    __shared__ long long s_pos[kChunk];
+    __shared__ double s_v[kChunk];
+    __shared__ unsigned s_t[kChunk];
+    __shared__ unsigned s_first[64];  // smallest sequence number of the lane's entries
+    __shared__ int s_count[64], s_base[64];
+    const unsigned c = blockIdx.x;
+    const int s = threadIdx.x;
+    const int fill = pool.fill()[c];
+    if (s < 64) {
+        s_first[s] = ~0u;
+        s_count[s] = 0;
+    }
+    __syncthreads();
+    PeakEntry e{};
+    const bool has = s < fill;
+    if (has) {
+        e = pool.entries[(size_t)c * kChunk + s];
+        atomicMin(&s_first[e.kl & 63u], e.kl >> 6);
+        atomicAdd(&s_count[e.kl & 63u], 1);
+    }
+    __syncthreads();
+    if (s < 64) {
+        const int own = s_count[s];
+        int x = own;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o);
+            if (s >= o) x += y;
+        }
+        s_base[s] = x - own;
+    }
+    __syncthreads();
+    if (has) {
+        const int lane = e.kl & 63u;
+        const long long p = (long long)pool.owner()[c] * 64 + lane;
+        const int slot = s_base[lane] + (int)((e.kl >> 6) - s_first[lane]);
+        s_pos[slot] = p < n && flags[p] == 1 ? off[p] + (e.kl >> 6) : -1;
+        s_v[slot] = e.v;
+        if (times) s_t[slot] = e.t;
+    }
+    __syncthreads();
+    if (!has || s_pos[s] < 0) return;
+    if (vals) vals[s_pos[s]] = s_v[s];
+    if (times) times[s_pos[s]] = s_t[s];
 }
 
 void PeakPoolBuf::alloc(hipStream_t st, long long chunks)
@@ -224,9 +265,8 @@ bool bif_post(CallCtx& ctx, BifDevice& R, PeakPoolBuf& pool)
     else R.times.release();
     if (used > (unsigned)pool.nchunks) used = (unsigned)pool.nchunks;
     if (used > 0) {
-        hipLaunchKernelGGL(scatter_kernel, dim3(ceil_div((unsigned long long)used * kChunk, 256)), dim3(256), 0,
-                           ctx.stream(), pool.view(), used, R.flags.get(), R.off.get(), R.vals.get(), R.times.get(),
-                           n);
+        hipLaunchKernelGGL(scatter_kernel, dim3(used), dim3(kChunk), 0, ctx.stream(), pool.view(), R.flags.get(),
+                           R.off.get(), R.vals.get(), R.times.get(), n);
         CHAOS_HIP(hipGetLastError());
     }
     ctx.add_analysis_ms(ctx.end());
