@@ -281,7 +281,7 @@ void launch_lle_rows(CallCtx& ctx, int system, LleArgs p, long long row0, long l
     const int block = ctx.opt().block > 0 ? ctx.opt().block : 256;
     CHAOS_REQUIRE(block % 64 == 0 && block <= 256, "block must be a multiple of 64 and <= 256");
     const long long groups = (p.n_points + 63) / 64, simds = device_simds(ctx);
-    const long long windows = (long long)p.W * p.NTp, total = (long long)p.S + windows;
+    const long long windows = lle_window_ticks(p.S, p.W, p.NTp), total = (long long)p.S + windows;
     if (lle_split(groups, simds, windows)) {
         launch_lle_split(ctx, system, p, block, d_out);
         return;

@@ -58,6 +58,14 @@ inline long long rotate_chunk_ticks(long long ticks, long long unit)
     return (c + unit - 1) / unit * unit;
 }
 
+// Window ticks of an exponent map, for the rules on it: none for a transient of
+// negative length, whose run LleProg::ticks refuses (the map is 0), so such a
+// call keeps to the plain kernel, which asks LleProg::ticks.
+inline long long lle_window_ticks(long long S, long long W, long long NTp)
+{
+    return S < 0 ? 0 : W * NTp;
+}
+
 // Exponent maps: whether the windows run with the base and the perturbed
 // trajectory of a point on two neighbouring lanes instead of one after the
 // other on the same lane.  That halves each wavefront's instructions and

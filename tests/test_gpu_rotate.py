@@ -76,3 +76,14 @@ def test_rotating_basins_equal_served_job(chaos, sem, n):
     srv.close()
     assert np.array_equal(fl, fl2) and np.array_equal(feat, feat2)
     assert np.array_equal(lab, lab2)
+
+
+# A transient of negative length is refused by the lane program: the map is 0
+# at every size, also where small maps run on lane pairs and larger ones rotate.
+@pytest.mark.parametrize("sem", [0, 1])
+@pytest.mark.parametrize("n", [1, 5, 128, 200, 260])
+def test_negative_transient_gives_a_zero_map_at_every_size(chaos, sem, n):
+    print(f"negative transient n={n} sem={sem}", flush=True)
+    got = chaos.lle2d(250.0, 0.5, n, 0.01, 1e-7, ROS["ic"], ROS["ranges"], ROS["idx"], -1.0, ROS["values"],
+                      system="rossler_rk4", semantics=sem)
+    assert np.array_equal(got, np.zeros((n, n)))
