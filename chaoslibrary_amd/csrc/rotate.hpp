@@ -118,7 +118,8 @@ __device__ __forceinline__ void rotate(const RotateCtl& args, Body&& body)
 }
 
 // Control block in call scratch, cleared on the call's stream (a kernel, not a
-// memset); its error word is checked when the call finishes.
+// memset); its error word is checked at the end of the timed region
+// (CallCtx::end).
 RotateCtl make_rotate_ctl(CallCtx& ctx, long long groups, long long chunks);
 // Blocks of 256 threads that put `waves` wavefronts on every SIMD.
 unsigned rotate_grid(CallCtx& ctx, int waves);

@@ -292,6 +292,7 @@ double CallCtx::end()
     CHAOS_HIP(hipEventSynchronize(ev1_));
     float ms = 0;
     CHAOS_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
+    check_watched();  // before anything reads what the region's launches wrote
     return ms;
 }
 

@@ -131,7 +131,7 @@ public:
     // Timed region on the call stream: begin() ... end() adds device ms to
     // the named accumulator of chaos_stats.
     void begin();
-    double end();            // returns ms of this region (synchronises)
+    double end();            // returns ms of this region (synchronises; fails on a watched word)
     void sync();
     // Device scratch of the call's launches, one block per slot: kept for the
     // call's next launch (its launches follow each other on one stream), grown
@@ -143,9 +143,11 @@ public:
     void add_steps(double s) { steps_ += s; }
     void add_launch(int n = 1) { launches_ += n; }
     void add_peaks(long long n) { peaks_ += n; }
-    // A device error word of the launches so far: finish() fails the call when
-    // it is not 0 (the word must live as long as the context; check_watched()
-    // reads it now, before the word is used anew).
+    // A device error word of the launches so far, in memory that lives as long
+    // as the context.  One that is not 0 fails the call at the end() of the
+    // launches' region, before the next stage indexes with outputs that were
+    // never written; check_watched() looks now (before the word is used anew),
+    // finish() for launches outside a region.
     void watch(const int* word) { watched_ = word; }
     void check_watched();
     void finish();          // fill opt.stats
