@@ -58,6 +58,7 @@ __global__ __launch_bounds__(kChunk) void scatter_kernel(const PeakPool pool, co
         s_first[s] = ~0u;
         s_count[s] = 0;
     }
+    s_pos[s] = -1;
     __syncthreads();
     PeakEntry e{};
     const bool has = s < fill;
@@ -79,11 +80,13 @@ __global__ __launch_bounds__(kChunk) void scatter_kernel(const PeakPool pool, co
     __syncthreads();
     if (has) {
         const int lane = e.kl & 63u;
-        const long long p = (long long)pool.owner()[c] * 64 + lane;
-        const int slot = s_base[lane] + (int)((e.kl >> 6) - s_first[lane]);
-        s_pos[slot] = p < n && flags[p] == 1 ? off[p] + (e.kl >> 6) : -1;
-        s_v[slot] = e.v;
-        if (times) s_t[slot] = e.t;
+        const long long p = (long long)(unsigned)pool.owner()[c] * 64 + lane;
+        const int place = chunk_place(s_base[lane], s_count[lane], s_first[lane], e.kl >> 6);
+        if (place >= 0) {
+            s_pos[place] = p < n && flags[p] == 1 ? off[p] + (e.kl >> 6) : -1;
+            s_v[place] = e.v;
+            if (times) s_t[place] = e.t;
+        }
     }
     __syncthreads();
     if (!has || s_pos[s] < 0) return;

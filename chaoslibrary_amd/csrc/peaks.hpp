@@ -224,6 +224,15 @@ struct PeakPool {
     __host__ __device__ int* overflow() const { return meta + 2 * (size_t)nchunks + 1; }  // pool ran out
 };
 
+// Place in its chunk of an entry with sequence number seq, the chunk put in
+// order of (lane, sequence): the lane's entries take the `count` places from
+// `base`, consecutive from the smallest sequence number `first`.  -1 for an
+// entry that is not one of them, as a chunk that no wave filled may hold.
+__host__ __device__ inline int chunk_place(int base, int count, unsigned first, unsigned seq)
+{
+    return seq - first < (unsigned)count ? base + (int)(seq - first) : -1;
+}
+
 struct WaveCursor {
     unsigned chunk;  // current chunk (nchunks when none / exhausted)
     int fill;        // entries used in it
