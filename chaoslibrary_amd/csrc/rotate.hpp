@@ -64,9 +64,15 @@ constexpr unsigned kRotatePolls = 1u << 27;
 // reports the call as failed.  The state crosses the XCDs' L2 caches between
 // chunks: parked and released at agent scope, acquired before it is loaded.
 //
-// Lane 0 takes the ticket for the wave, so the lanes must come to it together:
-// every trip ends in a wave barrier, which keeps lanes that skip a divergent
-// tail of the body (or of the hand-over) from taking the back edge on their own.
+// Lane 0 takes the ticket for the wave, so the lanes must come to it together.
+// Every trip ends in a wave barrier: the compiler may not put it under a further
+// condition, so lanes that skip a divergent tail of the body meet the others
+// there before the back edge.  That is how it treats the barrier, not something
+// the barrier promises, so each trip begins by looking at which lanes are
+// active: a wavefront that is not whole sets the error word and leaves, and the
+// call fails instead of taking a ticket with some of its lanes.  (An earlier
+// form ended the loop in `if (lane == 0) store`; the other lanes took the back
+// edge alone and read ticket 0 for ever.)
 template <class Body>
 __device__ __forceinline__ void rotate(const RotateCtl& args, Body&& body)
 {
@@ -78,6 +84,10 @@ __device__ __forceinline__ void rotate(const RotateCtl& args, Body&& body)
     unsigned trip = 0;
     for (;;) {
         const RotateCtl ctl = kept.get();
+        if (__builtin_amdgcn_ballot_w64(true) != ~0ull) {
+            __hip_atomic_store(ctl.err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
+        }
         const unsigned total = ctl.groups * ctl.chunks;
         // one ticket a wave: lane 0 takes it (the lanes are together here).  An
         // add by all 64 lanes would hand out 64 numbers, which are one atomic

@@ -1,0 +1,23 @@
+"""The rotating kernels check that a wavefront's 64 lanes are together where it
+takes a ticket (rotate.hpp); the check is in the built code of every one."""
+import os
+import re
+
+import pytest
+
+from test_build_guard import BUILD, LLVM, _device_asm
+
+
+@pytest.mark.parametrize("obj,kernels", [("lle.o", ["lle_rotate_kernel", "lle_pair_rotate_kernel"]),
+                                         ("sweep_rotate.o", ["sweep_rotate_kernel"])])
+def test_rotating_kernels_check_for_whole_wavefronts(tmp_path, obj, kernels):
+    path = os.path.join(BUILD, obj)
+    if not os.path.exists(path) or not os.path.exists(f"{LLVM}/llvm-objdump"):
+        pytest.skip("no built objects or no ROCm LLVM tools")
+    asm = _device_asm(path, str(tmp_path))
+    bodies = re.split(r"\n[0-9a-f]+ <(\w+)>:\n", asm)[1:]
+    for kernel in kernels:
+        found = [(n, b) for n, b in zip(bodies[::2], bodies[1::2]) if kernel in n]
+        assert len(found) >= 7
+        for name, body in found:
+            assert re.search(r"\bs_cmp_(eq|lg)_u64 exec, -1\b", body), name
