@@ -1,5 +1,6 @@
-"""The rotating kernels check that a wavefront's 64 lanes are together where it
-takes a ticket (rotate.hpp); the check is in the built code of every one."""
+"""Active lanes in the built code: the rotating kernels check that a wavefront's
+64 lanes are together where it takes a ticket (rotate.hpp), and the sweeps'
+masked moves (lanes.hpp) do not assume which lanes are active."""
 import os
 import re
 
@@ -21,3 +22,14 @@ def test_rotating_kernels_check_for_whole_wavefronts(tmp_path, obj, kernels):
         assert len(found) >= 7
         for name, body in found:
             assert re.search(r"\bs_cmp_(eq|lg)_u64 exec, -1\b", body), name
+
+
+# The sweeps move pending peaks under a lane mask written to exec; the lanes
+# that were active come back from a saved copy, not from "all 64".
+@pytest.mark.parametrize("obj", ["sweep.o", "sweep_rotate.o", "engine.o"])
+def test_sweeps_restore_the_active_lanes_they_had(tmp_path, obj):
+    path = os.path.join(BUILD, obj)
+    if not os.path.exists(path) or not os.path.exists(f"{LLVM}/llvm-objdump"):
+        pytest.skip("no built objects or no ROCm LLVM tools")
+    asm = _device_asm(path, str(tmp_path))
+    assert not re.search(r"\bs_mov_b64 exec, -1\b", asm)
