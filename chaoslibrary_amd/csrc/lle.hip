@@ -245,7 +245,8 @@ static double* lane_state(CallCtx& ctx, int nd, long long groups)
 static void launch_lle_split(CallCtx& ctx, int system, const LleArgs& p, int block, double* d_out)
 {
     const long long n = p.n_points, pairs = (2 * n + 63) / 64;
-    const int turn = rotate_waves(ROTATE_LLE, pairs, device_simds(ctx), (long long)p.W * p.NTp);
+    const long long windows = (long long)p.W * p.NTp;
+    const int turn = rotate_waves(ROTATE_LLE, pairs, device_simds(ctx), windows, p.NTp, 1);
     dispatch_system(system, [&](auto tag) {
         constexpr int S = decltype(tag)::value;
         constexpr int NX = System<S>::NX;
@@ -260,7 +261,7 @@ static void launch_lle_split(CallCtx& ctx, int system, const LleArgs& p, int blo
             ctx.add_launch();
         }
         if (turn) {
-            const int chunk = (int)(rotate_chunk_ticks((long long)p.W * p.NTp, p.NTp) / p.NTp);
+            const int chunk = (int)(rotate_chunk_ticks(windows, p.NTp, 1) / p.NTp);
             const RotateCtl ctl = make_rotate_ctl(ctx, pairs, (p.W + chunk - 1) / chunk);
             const LaneStore st{mem + NX * xn, nullptr, xn};
             hipLaunchKernelGGL(lle_pair_rotate_kernel<S>, dim3(rotate_grid(ctx, turn)), dim3(256), 0, ctx.stream(), p,
@@ -286,11 +287,11 @@ void launch_lle_rows(CallCtx& ctx, int system, LleArgs p, long long row0, long l
         launch_lle_split(ctx, system, p, block, d_out);
         return;
     }
-    const int turn = rotate_waves(ROTATE_LLE, groups, simds, total);
+    const int turn = rotate_waves(ROTATE_LLE, groups, simds, total, 1, 2);
     dispatch_system(system, [&](auto tag) {
         constexpr int S = decltype(tag)::value;
         if (turn) {
-            const long long chunk = rotate_chunk_ticks(total, 1);
+            const long long chunk = rotate_chunk_ticks(total, 1, 2);
             const RotateCtl ctl = make_rotate_ctl(ctx, groups, (total + chunk - 1) / chunk);
             const LaneStore st{lane_state(ctx, LleProg<S>::ND, groups), nullptr, groups * 64};
             hipLaunchKernelGGL(lle_rotate_kernel<S>, dim3(rotate_grid(ctx, turn)), dim3(256), 0, ctx.stream(), p, ctl,

@@ -1,5 +1,6 @@
 // rotate.hip -- host side of the rotating launches (rotate.hpp).
 #include "rotate.hpp"
+#include "rotate_plan.hpp"
 
 namespace chaos {
 
@@ -11,7 +12,7 @@ __global__ void rotate_clear_kernel(unsigned* p, unsigned n)
 
 RotateCtl make_rotate_ctl(CallCtx& ctx, long long groups, long long chunks)
 {
-    CHAOS_REQUIRE(groups > 0 && chunks > 0 && groups * chunks < (1LL << 25), "rotating launch too large");
+    CHAOS_REQUIRE(groups > 0 && chunks > 0 && groups * chunks < kRotateTickets, "rotating launch too large");
     ctx.check_watched();  // an earlier launch of this call used the same block
     // the ticket counter and the error word on a cache line of their own
     constexpr unsigned kPad = 32;

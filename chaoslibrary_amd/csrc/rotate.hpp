@@ -52,7 +52,8 @@ struct InVgprs {
     }
 };
 
-// Polls of a wait before it is given up (a poll takes about a microsecond).
+// Polls of a wait before it is given up (a poll takes 0.5 to 1 us; the chunk
+// waited for takes 10 s at most, kRotateChunkSteps).
 constexpr unsigned kRotatePolls = 1u << 27;
 
 // body(group, chunk, lane) for every ticket.  A ticket's predecessor (the same

@@ -12,6 +12,27 @@ enum RotateKind { ROTATE_LLE, ROTATE_SWEEP };
 
 constexpr long long kRotateChunk = 2000;  // fewest ticks per chunk
 constexpr int kRotateMinChunks = 12, kRotateMaxChunks = 48;
+// Most steps of a trajectory in a chunk, and tickets (groups * chunks) in a run.
+// A wavefront waits for the chunk before its own and gives up after about a
+// minute or two (kRotatePolls, rotate.hpp), which must mean that the chunk's
+// wavefront is gone and not that the run is a long one: a step is at most 4 us
+// (the slowest map, two trajectories a lane, two wavefronts on the SIMD), so a
+// chunk stays below 10 s.
+constexpr long long kRotateChunkSteps = 1LL << 21, kRotateTickets = 1LL << 25;
+
+// Ticks per chunk: a run of `ticks` in at most kRotateMaxChunks chunks of at
+// least kRotateChunk ticks, rounded up to a multiple of `unit`; more chunks, of
+// one unit or more, where `steps` steps a tick (0: not asked) would make that
+// more than kRotateChunkSteps steps.
+inline long long rotate_chunk_ticks(long long ticks, long long unit, long long steps = 0)
+{
+    long long c = (ticks + kRotateMaxChunks - 1) / kRotateMaxChunks;
+    if (c < kRotateChunk) c = kRotateChunk;
+    if (unit < 1) unit = 1;
+    c = (c + unit - 1) / unit;
+    if (steps > 0 && c > kRotateChunkSteps / steps / unit) c = kRotateChunkSteps / steps / unit;
+    return c < 1 ? unit : c * unit;
+}
 
 // Wavefronts per SIMD of a rotating launch (rotate.hpp) over `groups`
 // wavefronts of work, or 0 to launch them all at once.
@@ -33,11 +54,16 @@ constexpr int kRotateMinChunks = 12, kRotateMaxChunks = 48;
 // wavefronts a SIMD (the most that reside: the hardware's refill evens the
 // load), and for runs of fewer than 12 chunks of 2000 ticks (`ticks` per
 // group): shorter chunks cost too much to hand over and fewer leave an uneven
-// end of their own.
-inline int rotate_waves(RotateKind kind, long long groups, long long simds, long long ticks)
+// end of their own.  It stays, too, where the chunks (of `unit` ticks or more)
+// would be too long to wait for or too many.
+inline int rotate_waves(RotateKind kind, long long groups, long long simds, long long ticks, long long unit = 1,
+                        long long steps = 0)
 {
     if (simds <= 0 || groups <= simds || groups > 8 * simds) return 0;
     if (ticks < kRotateChunk * kRotateMinChunks) return 0;
+    const long long chunk = rotate_chunk_ticks(ticks, unit, steps), chunks = (ticks + chunk - 1) / chunk;
+    if (steps > 0 && chunk > kRotateChunkSteps / steps) return 0;
+    if (chunks >= kRotateTickets / groups) return 0;
     const double w = (double)groups / (double)simds;
     const double c = (double)((groups + simds - 1) / simds);
     const double at_once = kind == ROTATE_LLE ? c : c + 0.34;
@@ -46,16 +72,6 @@ inline int rotate_waves(RotateKind kind, long long groups, long long simds, long
     const double best = one < two ? one : two;
     if (best >= 0.98 * at_once) return 0;
     return one < two ? 1 : 2;
-}
-
-// Ticks per chunk: a run of `ticks` in at most kRotateMaxChunks chunks of at
-// least kRotateChunk ticks, rounded up to a multiple of `unit`.
-inline long long rotate_chunk_ticks(long long ticks, long long unit)
-{
-    long long c = (ticks + kRotateMaxChunks - 1) / kRotateMaxChunks;
-    if (c < kRotateChunk) c = kRotateChunk;
-    if (unit < 1) unit = 1;
-    return (c + unit - 1) / unit * unit;
 }
 
 // Window ticks of an exponent map, for the rules on it: none for a transient of

@@ -82,7 +82,7 @@ void launch_sweep(CallCtx& ctx, int system, int writableVar, int kind, const Swe
     chaos_system_dims(system, &nx, &na);
     CHAOS_REQUIRE(writableVar >= 0 && writableVar < nx, "writableVar %d out of range [0,%d)", writableVar, nx);
     if (const int turn = rotate_waves(ROTATE_SWEEP, ceil_div((unsigned long long)A.n_points, 64), device_simds(ctx),
-                                      (long long)A.S + A.B)) {
+                                      (long long)A.S + A.B, 1, A.pre)) {
         launch_sweep_rotating(ctx, system, writableVar, kind, A, turn);
         return;
     }

@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256) void feature_moments_kernel(const SweepArgs A)
 void launch_sweep_rotating(CallCtx& ctx, int system, int writableVar, int kind, const SweepArgs& A, int waves)
 {
     const long long groups = (A.n_points + 63) / 64, np = groups * 64;
-    const long long total = (long long)A.S + A.B, chunk = rotate_chunk_ticks(total, 1);
+    const long long total = (long long)A.S + A.B, chunk = rotate_chunk_ticks(total, 1, A.pre);
     const RotateCtl ctl = make_rotate_ctl(ctx, groups, (total + chunk - 1) / chunk);
     dispatch_system(system, [&](auto tag) {
         constexpr int S = decltype(tag)::value;
