@@ -54,7 +54,11 @@ inline long long rotate_chunk_ticks(long long ticks, long long unit, long long s
 // wavefronts a SIMD (the most that reside: the hardware's refill evens the
 // load), and for runs of fewer than 12 chunks of 2000 ticks (`ticks` per
 // group): shorter chunks cost too much to hand over and fewer leave an uneven
-// end of their own.  It stays, too, where the chunks (of `unit` ticks or more)
+// end of their own.  Chunks of one long `unit` each may be fewer; the rounds in
+// which they are run then count whole (lane pairs on 1.22 and 1.76 wavefronts a
+// SIMD, 40,000 window ticks, at once / in turns: one window 6.15 / 6.21 and 5.82
+// / 6.16 ms, two 6.14 / 4.84 and 5.84 / 6.23, four 5.99 / 3.97 and 5.81 / 6.16,
+// six 5.97 / 4.18 and 5.83 / 5.70).  The plain launch stays, too, where the chunks
 // would be too long to wait for or too many.
 inline int rotate_waves(RotateKind kind, long long groups, long long simds, long long ticks, long long unit = 1,
                         long long steps = 0)
@@ -64,11 +68,16 @@ inline int rotate_waves(RotateKind kind, long long groups, long long simds, long
     const long long chunk = rotate_chunk_ticks(ticks, unit, steps), chunks = (ticks + chunk - 1) / chunk;
     if (steps > 0 && chunk > kRotateChunkSteps / steps) return 0;
     if (chunks >= kRotateTickets / groups) return 0;
-    const double w = (double)groups / (double)simds;
+    const long long units = groups * chunks;
+    double w = (double)groups / (double)simds, w2 = w;
+    if (chunks < kRotateMinChunks) {
+        w = (double)((units + simds - 1) / simds) / (double)chunks;
+        w2 = 2.0 * (double)((units + 2 * simds - 1) / (2 * simds)) / (double)chunks;
+    }
     const double c = (double)((groups + simds - 1) / simds);
     const double at_once = kind == ROTATE_LLE ? c : c + 0.34;
     const double one = kind == ROTATE_LLE ? 1.03 * w : 1.33 * w;
-    const double two = groups < 2 * simds ? 1e30 : kind == ROTATE_LLE ? 0.92 * w + 0.6 : w + 0.38;
+    const double two = groups < 2 * simds ? 1e30 : kind == ROTATE_LLE ? 0.92 * w2 + 0.6 : w2 + 0.38;
     const double best = one < two ? one : two;
     if (best >= 0.98 * at_once) return 0;
     return one < two ? 1 : 2;

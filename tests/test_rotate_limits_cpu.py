@@ -53,3 +53,15 @@ def test_long_runs_keep_a_plan(lib):
     assert lib.plan_waves(0, 1407, SIMDS, 2 ** 31, 50, 1) == 1
     assert lib.plan_waves(1, 1407, SIMDS, 2 ** 31, 1, 1) == 1
     assert lib.plan_waves(1, 1407, SIMDS, 2 ** 31, 1, 10 ** 6) == 0
+
+
+# Few chunks, of one long window each: taken in turns only where the whole
+# rounds they need are fewer than the wavefronts of the fullest SIMD.
+@pytest.mark.parametrize("groups", [1025, 1250, 1407, 1800, 2047])
+def test_few_long_chunks_count_whole_rounds(lib, groups):
+    unit = 40000
+    for windows in range(1, 12):
+        rounds = -(-groups * windows // SIMDS)
+        got = lib.plan_waves(0, groups, SIMDS, windows * unit, unit, 1)
+        assert got == (1 if 1.03 * rounds / windows < 0.98 * 2 else 0), windows
+    assert lib.plan_waves(0, groups, SIMDS, unit, unit, 1) == 0
