@@ -241,6 +241,24 @@ static double* lane_state(CallCtx& ctx, int nd, long long groups)
     return static_cast<double*>(ctx.scratch(CallCtx::SCRATCH_STATE, (size_t)nd * groups * 64 * sizeof(double)));
 }
 
+// lle_split's measured costs: the steps a window's end takes, and the time of
+// two wavefronts on a SIMD at once with one trajectory a lane over that of one
+// wavefront with two.  The long steps of BASINS and DAMIR, with their sines and
+// exponentials, leave a lone wavefront waiting (DAMIR 240^2, 2000 window ticks
+// in windows of 1 and 50 steps, on one lane / on pairs: 8.0 / 7.3, 7.0 / 5.6 ms).
+template <int SYS>
+struct PairCost {
+    static constexpr double end = 4.0, two = 1.0;
+};
+template <>
+struct PairCost<SYS_BASINS> {
+    static constexpr double end = 1.0, two = 0.92;
+};
+template <>
+struct PairCost<SYS_DAMIR> {
+    static constexpr double end = 0.5, two = 0.8;
+};
+
 // Transient on one lane per point, then the windows on lane pairs.
 static void launch_lle_split(CallCtx& ctx, int system, const LleArgs& p, int block, double* d_out)
 {
@@ -283,7 +301,12 @@ void launch_lle_rows(CallCtx& ctx, int system, LleArgs p, long long row0, long l
     CHAOS_REQUIRE(block % 64 == 0 && block <= 256, "block must be a multiple of 64 and <= 256");
     const long long groups = (p.n_points + 63) / 64, simds = device_simds(ctx);
     const long long windows = lle_window_ticks(p.S, p.W, p.NTp), total = (long long)p.S + windows;
-    if (lle_split(groups, simds, windows)) {
+    bool split = false;
+    dispatch_system(system, [&](auto tag) {
+        using Cost = PairCost<decltype(tag)::value>;
+        split = lle_split(groups, simds, windows, p.NTp, Cost::end, Cost::two);
+    });
+    if (split) {
         launch_lle_split(ctx, system, p, block, d_out);
         return;
     }

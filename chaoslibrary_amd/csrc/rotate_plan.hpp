@@ -60,27 +60,40 @@ inline long long rotate_chunk_ticks(long long ticks, long long unit, long long s
 // / 6.16 ms, two 6.14 / 4.84 and 5.84 / 6.23, four 5.99 / 3.97 and 5.81 / 6.16,
 // six 5.97 / 4.18 and 5.83 / 5.70).  The plain launch stays, too, where the chunks
 // would be too long to wait for or too many.
-inline int rotate_waves(RotateKind kind, long long groups, long long simds, long long ticks, long long unit = 1,
-                        long long steps = 0)
+struct RotatePlan {
+    int waves;    // wavefronts per SIMD, 0: all at once
+    double time;  // in the units above
+};
+
+inline RotatePlan rotate_plan(RotateKind kind, long long groups, long long simds, long long ticks, long long unit,
+                              long long steps)
 {
-    if (simds <= 0 || groups <= simds || groups > 8 * simds) return 0;
-    if (ticks < kRotateChunk * kRotateMinChunks) return 0;
+    if (simds <= 0) return {0, 1e30};
+    const double c = (double)((groups + simds - 1) / simds);
+    const double at_once = kind == ROTATE_LLE ? c : c + 0.34;
+    const RotatePlan plain{0, at_once};
+    if (groups <= simds || groups > 8 * simds) return plain;
+    if (ticks < kRotateChunk * kRotateMinChunks) return plain;
     const long long chunk = rotate_chunk_ticks(ticks, unit, steps), chunks = (ticks + chunk - 1) / chunk;
-    if (steps > 0 && chunk > kRotateChunkSteps / steps) return 0;
-    if (chunks >= kRotateTickets / groups) return 0;
+    if (steps > 0 && chunk > kRotateChunkSteps / steps) return plain;
+    if (chunks >= kRotateTickets / groups) return plain;
     const long long units = groups * chunks;
     double w = (double)groups / (double)simds, w2 = w;
     if (chunks < kRotateMinChunks) {
         w = (double)((units + simds - 1) / simds) / (double)chunks;
         w2 = 2.0 * (double)((units + 2 * simds - 1) / (2 * simds)) / (double)chunks;
     }
-    const double c = (double)((groups + simds - 1) / simds);
-    const double at_once = kind == ROTATE_LLE ? c : c + 0.34;
     const double one = kind == ROTATE_LLE ? 1.03 * w : 1.33 * w;
     const double two = groups < 2 * simds ? 1e30 : kind == ROTATE_LLE ? 0.92 * w2 + 0.6 : w2 + 0.38;
     const double best = one < two ? one : two;
-    if (best >= 0.98 * at_once) return 0;
-    return one < two ? 1 : 2;
+    if (best >= 0.98 * at_once) return plain;
+    return {one < two ? 1 : 2, best};
+}
+
+inline int rotate_waves(RotateKind kind, long long groups, long long simds, long long ticks, long long unit = 1,
+                        long long steps = 0)
+{
+    return rotate_plan(kind, groups, simds, ticks, unit, steps).waves;
 }
 
 // Window ticks of an exponent map, for the rules on it: none for a transient of
@@ -93,15 +106,27 @@ inline long long lle_window_ticks(long long S, long long W, long long NTp)
 
 // Exponent maps: whether the windows run with the base and the perturbed
 // trajectory of a point on two neighbouring lanes instead of one after the
-// other on the same lane.  That halves each wavefront's instructions and
-// doubles the wavefronts: a gain while SIMDs are without one (17^2 points, 2100
-// window ticks: 384 -> 251 us; Rossler with half its 80,000 ticks in windows
-// 128^2 9.2 -> 6.4 ms, 200^2 9.3 -> 7.6, 230^2 (0.81 wavefronts per SIMD) 9.2 ->
-// 8.8), none when they are full (256^2: 9.7 -> 10.0, so the line is at 0.9).
-// window_ticks = W * NTp: below 200 the second launch costs what it saves.
-inline bool lle_split(long long groups, long long simds, long long window_ticks)
+// other on the same lane.  That halves each wavefront's steps and doubles the
+// wavefronts.  Both lanes do a window's end (the distance and its logarithm), so
+// a wavefront's work falls to (NTp + end) / (2 NTp + end), `end` in steps; up to
+// one wavefront of pairs a SIMD that is the gain (17^2 points, 2100 window
+// ticks: 384 -> 251 us; Rossler with half its 80,000 ticks in windows 128^2 9.2 ->
+// 6.4 ms).  Above, the SIMD does that work twice, which gains where the pairs'
+// wavefronts take turns (200^2 9.3 -> 7.6 ms, 230^2 (0.81 wavefronts per SIMD) 9.2
+// -> 8.8; none when the SIMDs are full, 256^2: 9.7 -> 10.0, so the line is at
+// 0.9), or where two wavefronts at once take `two` < 1 times the time of one with
+// both trajectories.  Too few ticks for turns, on one lane / on pairs:
+// 200^2 and 240^2 Rossler, 2000 window ticks in windows of 1, 8, 50 steps 1.50 /
+// 2.10, 0.84 / 1.01, 0.67 / 0.70 ms; BASINS in windows of 1, 4, 8, 50 steps
+// 2.9 / 3.4, 1.89 / 1.89, 1.80 / 1.71, 1.70 / 1.58.
+// Below 200 window ticks the second launch costs what it saves.
+inline bool lle_split(long long groups, long long simds, long long window_ticks, long long NTp, double end, double two)
 {
-    return simds > 0 && 10 * groups <= 9 * simds && window_ticks >= 200;
+    if (simds <= 0 || 10 * groups > 9 * simds || window_ticks < 200) return false;
+    const long long pairs = 2 * groups;
+    const RotatePlan plan = rotate_plan(ROTATE_LLE, pairs, simds, window_ticks, NTp, 1);
+    const double time = plan.waves || pairs <= simds ? plan.time : two * plan.time;
+    return time * ((double)NTp + end) / (2.0 * (double)NTp + end) < 0.98;
 }
 
 }  // namespace chaos

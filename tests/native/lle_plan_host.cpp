@@ -4,7 +4,7 @@
 
 extern "C" int lle_split_host(long long groups, long long simds, long long S, long long W, long long NTp)
 {
-    return chaos::lle_split(groups, simds, chaos::lle_window_ticks(S, W, NTp));
+    return chaos::lle_split(groups, simds, chaos::lle_window_ticks(S, W, NTp), NTp, 4.0, 1.0);
 }
 
 extern "C" int lle_turn_host(long long groups, long long simds, long long S, long long W, long long NTp)

@@ -33,3 +33,18 @@ def test_a_refused_run_keeps_the_plain_kernel(lib, groups):
         assert not lib.lle_turn_host(groups, SIMDS, S, 1000, 50)
     assert lib.lle_split_host(groups, SIMDS, 0, 1000, 50) == (groups <= 900)
     assert (lib.lle_turn_host(groups, SIMDS, 0, 1000, 50) > 0) == (groups > SIMDS)
+
+
+# Lane pairs double the work of a window's end: above one wavefront of pairs a
+# SIMD they are taken only where turns make up for it, so neither for windows of
+# a few steps nor for runs too short for turns.
+def test_short_windows_and_short_runs_stay_on_one_lane(lib):
+    for groups in (520, 625, 900):
+        for NTp in (1, 2, 4, 8, 16, 50, 100):
+            assert not lib.lle_split_host(groups, SIMDS, 500, 20000 // NTp, NTp)
+    assert not lib.lle_split_host(625, SIMDS, 500, 40000, 1)
+    assert lib.lle_split_host(625, SIMDS, 500, 800, 50)
+    for groups in (1, 100, 512):
+        for NTp in (1, 50):
+            assert lib.lle_split_host(groups, SIMDS, 500, 200 // NTp, NTp)
+            assert not lib.lle_split_host(groups, SIMDS, 500, 199 // NTp, NTp)
