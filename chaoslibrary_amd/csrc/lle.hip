@@ -282,8 +282,8 @@ static void launch_lle_split(CallCtx& ctx, int system, const LleArgs& p, int blo
             const int chunk = (int)(rotate_chunk_ticks(windows, p.NTp, 1) / p.NTp);
             const RotateCtl ctl = make_rotate_ctl(ctx, pairs, (p.W + chunk - 1) / chunk);
             const LaneStore st{mem + NX * xn, nullptr, xn};
-            hipLaunchKernelGGL(lle_pair_rotate_kernel<S>, dim3(rotate_grid(ctx, turn)), dim3(256), 0, ctx.stream(), p,
-                               ctl, chunk, xs, xn, st, d_out);
+            hipLaunchKernelGGL(lle_pair_rotate_kernel<S>, dim3(rotate_grid(ctx, turn, block)), dim3(block), 0,
+                               ctx.stream(), p, ctl, chunk, xs, xn, st, d_out);
         } else {
             hipLaunchKernelGGL(lle_pair_kernel<S>, dim3(ceil_div(2 * n, block)), dim3(block), 0, ctx.stream(), p, xs,
                                xn, d_out);
@@ -317,8 +317,8 @@ void launch_lle_rows(CallCtx& ctx, int system, LleArgs p, long long row0, long l
             const long long chunk = rotate_chunk_ticks(total, 1, 2);
             const RotateCtl ctl = make_rotate_ctl(ctx, groups, (total + chunk - 1) / chunk);
             const LaneStore st{lane_state(ctx, LleProg<S>::ND, groups), nullptr, groups * 64};
-            hipLaunchKernelGGL(lle_rotate_kernel<S>, dim3(rotate_grid(ctx, turn)), dim3(256), 0, ctx.stream(), p, ctl,
-                               chunk, st, d_out);
+            hipLaunchKernelGGL(lle_rotate_kernel<S>, dim3(rotate_grid(ctx, turn, block)), dim3(block), 0, ctx.stream(), p,
+                               ctl, chunk, st, d_out);
         } else {
             hipLaunchKernelGGL(lle_map_kernel<S>, dim3(ceil_div(p.n_points, block)), dim3(block), 0, ctx.stream(), p,
                                d_out);

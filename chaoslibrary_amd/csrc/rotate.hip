@@ -27,9 +27,9 @@ RotateCtl make_rotate_ctl(CallCtx& ctx, long long groups, long long chunks)
 
 long long device_simds(CallCtx& ctx) { return 4LL * device_props(ctx.device()).multiProcessorCount; }
 
-unsigned rotate_grid(CallCtx& ctx, int waves)
+unsigned rotate_grid(CallCtx& ctx, int waves, int block)
 {
-    return (unsigned)(device_props(ctx.device()).multiProcessorCount * waves);
+    return rotate_blocks(device_props(ctx.device()).multiProcessorCount, waves, block);
 }
 
 }  // namespace chaos

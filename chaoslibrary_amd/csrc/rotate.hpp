@@ -132,8 +132,8 @@ __device__ __forceinline__ void rotate(const RotateCtl& args, Body&& body)
 // memset); its error word is checked at the end of the timed region
 // (CallCtx::end).
 RotateCtl make_rotate_ctl(CallCtx& ctx, long long groups, long long chunks);
-// Blocks of 256 threads that put `waves` wavefronts on every SIMD.
-unsigned rotate_grid(CallCtx& ctx, int waves);
+// Blocks of `block` threads that put `waves` wavefronts on every SIMD.
+unsigned rotate_grid(CallCtx& ctx, int waves, int block = 256);
 // SIMDs of the call's device (four per CU).
 long long device_simds(CallCtx& ctx);
 

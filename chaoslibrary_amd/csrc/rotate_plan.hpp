@@ -96,6 +96,14 @@ inline int rotate_waves(RotateKind kind, long long groups, long long simds, long
     return rotate_plan(kind, groups, simds, ticks, unit, steps).waves;
 }
 
+// Blocks of `block` threads (a multiple of 64) that hold `waves` wavefronts for
+// each of a CU's four SIMDs; a wavefront takes tickets by itself, so the block's
+// size is the caller's choice.
+inline unsigned rotate_blocks(long long cus, int waves, int block)
+{
+    return (unsigned)((cus * waves * 256 + block - 1) / block);
+}
+
 // Window ticks of an exponent map, for the rules on it: none for a transient of
 // negative length, whose run LleProg::ticks refuses (the map is 0), so such a
 // call keeps to the plain kernel, which asks LleProg::ticks.

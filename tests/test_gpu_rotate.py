@@ -87,3 +87,19 @@ def test_negative_transient_gives_a_zero_map_at_every_size(chaos, sem, n):
     got = chaos.lle2d(250.0, 0.5, n, 0.01, 1e-7, ROS["ic"], ROS["ranges"], ROS["idx"], -1.0, ROS["values"],
                       system="rossler_rk4", semantics=sem)
     assert np.array_equal(got, np.zeros((n, n)))
+
+
+# The block size is the caller's choice on every path (plain, lane pairs,
+# rotating, rotating pairs) and changes nothing; what was refused is refused.
+@pytest.mark.parametrize("n,CT", [(17, 20.0), (60, 250.0), (200, 250.0), (260, 250.0)])
+def test_block_option_on_every_exponent_path(chaos, n, CT):
+    def run(block):
+        print(f"LLE n={n} CT={CT} block={block}", flush=True)
+        return chaos.lle2d(CT, 0.5, n, 0.01, 1e-7, ROS["ic"], ROS["ranges"], ROS["idx"], 5.0, ROS["values"],
+                           system="rossler_rk4", semantics=1, block=block)
+    want = run(0)
+    for block in (64, 128, 192, 256):
+        assert np.array_equal(run(block), want)
+    for block in (32, 100, 320):
+        with pytest.raises(Exception):
+            run(block)
