@@ -122,8 +122,8 @@ void engine_lle_kernel(const JobDev* __restrict__ jobs, const Tile* __restrict__
     });
 }
 
-// The sweep programs need up to 80 VGPRs here (lane state load/store on
-// top of the one-shot kernels' loop): 6 waves per SIMD, no spills.
+// The sweep programs need 68 to 80 VGPRs here (lane state load/store on top of
+// the one-shot kernels' loop): 6 waves per SIMD, no spills.
 template <int SYS, int KIND, int WV>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8)))
 void engine_sweep_kernel(const JobDev* __restrict__ jobs, const Tile* __restrict__ tiles, RoundCtl* __restrict__ ctl)

@@ -656,24 +656,30 @@ struct SweepProg {
         }
     }
 
+    // Parked state.  A kind parks what it uses: anything more stays in registers
+    // across the ticks between a load and the next store, and the engine's kernels
+    // have none to spare (all of it: 2 to 7 VGPRs spilled in the basins kernels).
+    // `last` and `fixed` are set by the record's last sample, after which nothing
+    // is parked.
+    static constexpr bool FIRST = BIF, SUMS = !BIF, MEANS = KIND == KIND_BASINS_CFG, LAST_T = KIND == KIND_BASINS_REF;
     __device__ __forceinline__ void load(const LaneStore& L, long long q)
     {
 #pragma unroll
         for (int k = 0; k < NX; ++k) X[k] = L.d[k * L.np + q];
         const double* d = L.d + NX * L.np + q;
         det.p = d[0];
-        first = d[L.np];
-        last = d[2 * L.np];
-        s0 = d[3 * L.np];
-        s1 = d[4 * L.np];
-        sx = d[5 * L.np];
-        sz = d[6 * L.np];
-        det.pstart = L.i[q];
+        first = FIRST ? d[L.np] : 0.0;
+        last = 0.0;
+        s0 = SUMS ? d[3 * L.np] : 0.0;
+        s1 = SUMS ? d[4 * L.np] : 0.0;
+        sx = MEANS ? d[5 * L.np] : 0.0;
+        sz = MEANS ? d[6 * L.np] : 0.0;
+        det.pstart = DET_TIMES ? L.i[q] : 0;
         cnt = L.i[L.np + q];
-        prev_t = L.i[2 * L.np + q];
+        prev_t = LAST_T ? L.i[2 * L.np + q] : 0;
         const int bits = L.i[3 * L.np + q];
         alive = wave_mask(bits & 1);
-        fixed = bits & 2;
+        fixed = false;
         det.m.plat = wave_mask(bits & 4);
         det.m.skip = wave_mask(bits & 8);
         det.m.up = wave_mask(bits & 16);
@@ -684,17 +690,20 @@ struct SweepProg {
         for (int k = 0; k < NX; ++k) L.d[k * L.np + q] = X[k];
         double* d = L.d + NX * L.np + q;
         d[0] = det.p;
-        d[L.np] = first;
-        d[2 * L.np] = last;
-        d[3 * L.np] = s0;
-        d[4 * L.np] = s1;
-        d[5 * L.np] = sx;
-        d[6 * L.np] = sz;
-        L.i[q] = det.pstart;
+        if (FIRST) d[L.np] = first;
+        if (SUMS) {
+            d[3 * L.np] = s0;
+            d[4 * L.np] = s1;
+        }
+        if (MEANS) {
+            d[5 * L.np] = sx;
+            d[6 * L.np] = sz;
+        }
+        if (DET_TIMES) L.i[q] = det.pstart;
         L.i[L.np + q] = cnt;
-        L.i[2 * L.np + q] = prev_t;
+        if (LAST_T) L.i[2 * L.np + q] = prev_t;
         L.i[3 * L.np + q] =
-            (lane_bit(alive) ? 1 : 0) | (fixed ? 2 : 0) | (lane_bit(det.m.plat) ? 4 : 0) |
+            (lane_bit(alive) ? 1 : 0) | (lane_bit(det.m.plat) ? 4 : 0) |
             (lane_bit(det.m.skip) ? 8 : 0) | (lane_bit(det.m.up) ? 16 : 0);
     }
 };
