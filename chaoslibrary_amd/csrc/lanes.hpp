@@ -455,7 +455,7 @@ struct SweepProg {
             else
                 for (int r = 0; r < A.pre; ++r) Sy::step(X, a, A.sc);
         };
-        unsigned long long busy = det.m.busy();
+        unsigned long long busy = det.m.busy() & alive;
         double p = det.p;
         unsigned long long up = det.m.up;
         unsigned long long pend = 0ull;  // lanes with a full slot (value pend_v, time pend_t)
@@ -463,44 +463,42 @@ struct SweepProg {
         int pend_t = 0;
         while (t + 1 < end) {
             double v0, v1;
-            unsigned long long c0, c1, y0, y1, o0, o1, other;
+            SamplePair m;
             do {
                 det.p = p;  // the history before the pair
                 det.m.up = up;
                 v0 = take<WVT>(wv);
                 const double d0 = v0 - p;
-                c0 = wave_mask(d0 <= 0.0);
-                y0 = wave_mask(fabs(d0) <= 1e-13);
-                o0 = wave_mask(!(fabs(v0) < A.L));
+                m.c0 = wave_mask(d0 <= 0.0);
+                m.y0 = wave_mask(fabs(d0) <= 1e-13);
+                m.o0 = wave_mask(!(fabs(v0) < A.L));
                 advance();
                 v1 = take<WVT>(wv);
                 const double d1 = v1 - v0;
-                c1 = wave_mask(d1 <= 0.0);
-                y1 = wave_mask(fabs(d1) <= 1e-13);
-                o1 = wave_mask(!(fabs(v1) < A.L));
-                // rising samples followed by one that does not rise
-                const unsigned long long f0 = up & c0, f1 = c1 & ~(c0 | y0);
-                other = ((o0 | o1) & alive) | busy;
+                m.c1 = wave_mask(d1 <= 0.0);
+                m.y1 = wave_mask(fabs(d1) <= 1e-13);
+                m.o1 = wave_mask(!(fabs(v1) < A.L));
+                const bool events = m.events(up, busy, alive);
                 advance();
                 pin_state();
                 t += 2;
-                if (f0 | f1 | other) {
-                    const unsigned long long e0 = f0 & ~y0 & alive, e1 = f1 & ~y1 & alive;
-                    other |= (f0 & y0) | (f1 & y1) | ((e0 | e1) & pend);
-                    if (other) break;
+                if (events) {
+                    unsigned long long e0, e1;
+                    m.peaks(alive, pend, e0, e1);
+                    if (m.other) break;
                     // the peaks are the samples t - 3 and t - 2 now
                     to_slots(pend_v, pend_t, p, t - 3, e0, v0, t - 2, e1);
                     pend |= e0 | e1;
                 }
                 p = v1;
-                up = ~(c1 | y1);
+                up = ~(m.c1 | m.y1);
             } while (t + 1 < end);
-            if (other) {
+            if (m.other) {
                 if (pend) on_peaks(A, cur, wave, pend, pend_v, pend_t);
                 pend = 0ull;
-                settle(A, cur, wave, t - 2, v0, c0, y0, o0);
-                settle(A, cur, wave, t - 1, v1, c1, y1, o1);
-                busy = det.m.busy();
+                settle(A, cur, wave, t - 2, v0, m.c0, m.y0, m.o0);
+                settle(A, cur, wave, t - 1, v1, m.c1, m.y1, m.o1);
+                busy = det.m.busy() & alive;
                 p = det.p;
                 up = det.m.up;
             }

@@ -147,6 +147,36 @@ struct PeakMasks {
     __host__ __device__ __forceinline__ unsigned long long busy() const { return plat | skip; }
 };
 
+// Two samples of a wave, one after the other, by their lane masks: c (not above
+// the sample before), y (within 1e-13 of it), o (outside the divergence band).
+// Says whether the pair is plain -- its peaks, if any, only join their lanes'
+// pending slots -- or goes sample by sample.  Lanes that no longer integrate
+// cannot make it do so: what their detector holds is never used.
+struct SamplePair {
+    unsigned long long c0, y0, o0, c1, y1, o1;
+    unsigned long long f0, f1;  // rising samples followed by one that does not rise
+    unsigned long long other;   // lanes for which the pair goes sample by sample
+
+    // `up` and `busy` are PeakMasks' before the pair, busy of lanes alive.
+    __host__ __device__ __forceinline__ bool events(unsigned long long up, unsigned long long busy,
+                                                    unsigned long long alive)
+    {
+        f0 = up & c0;
+        f1 = c1 & ~(c0 | y0);
+        other = ((o0 | o1) & alive) | busy;
+        return (f0 | f1 | other) != 0ull;
+    }
+    // The lanes with a peak at the pair's first (e0) and second sample (e1),
+    // where events() said that there may be any; pend: lanes whose slot is full.
+    __host__ __device__ __forceinline__ void peaks(unsigned long long alive, unsigned long long pend,
+                                                   unsigned long long& e0, unsigned long long& e1)
+    {
+        e0 = f0 & ~y0 & alive;
+        e1 = f1 & ~y1 & alive;
+        other |= (((f0 & y0) | (f1 & y1)) & alive) | ((e0 | e1) & pend);
+    }
+};
+
 // PeakDetector for a whole wave, as the sweeps use it: the masks, the last
 // sample's value and the plateau starts.  The compares are written into masks
 // and the emit mask feeds the wave's append directly.  All 64 lanes must take
