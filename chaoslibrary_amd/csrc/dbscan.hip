@@ -227,7 +227,7 @@ __device__ __forceinline__ int uf_load(const int* a) { return __hip_atomic_load(
 // compare-and-swap.  A table more than half full is flagged (the host redoes
 // the clustering with the larger table) and a search in it ends after eight
 // probes: nothing of the pass is used any more, and filled up, every insertion
-// would walk all of it (300,000 scattered points, a cell each: 10.9 s, 3.3 ms
+// would walk all of it (300,000 scattered points, a cell each: 10.9 s, 3.0 ms
 // so).
 __device__ __forceinline__ int hash_insert(const GridDev& G, unsigned long long key)
 {
@@ -390,8 +390,9 @@ constexpr int kAggGroups = 4;
 // Per-block chunks of the aggregated kernels: 256 threads x PER points,
 // consecutive point indices per pass, and an LDS table of kLds cells.  A long
 // chunk saves global atomics on the cells that many points share; a short one
-// fills the chip, and at PER = 1 the table holds every cell its 256 points can
-// lie in.  Whole clustering, 8 points a thread -> the rule below: 8,000 points
+// fills the chip, and at PER = 1 the table has twice as many entries as its 256
+// points can have cells (a key still goes to the global table when the 16 entries
+// from its place on are taken, kLdsProbes).  Whole clustering, 8 points a thread -> the rule below: 8,000 points
 // 0.24 -> 0.14 ms, 160,000 0.71 -> 0.65 ms, 300,000 1.07 -> 1.02 ms, the same
 // from 524,288 on.
 constexpr int kMaxPer = 8;

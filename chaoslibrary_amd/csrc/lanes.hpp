@@ -428,7 +428,7 @@ struct SweepProg {
     //
     // A peak needs a rising sample followed by a fall (up & c2 & ~tiny) and
     // nothing more unless a plateau is open or begins or an index is skipped;
-    // such a peak only joins its lane's pending slot (a masked move).  The slots
+    // such a peak only joins its lane's pending slot (to_slots).  The slots
     // are emptied together -- one append, or one masked update of the sums --
     // when a lane with a full slot peaks again: lanes peak every 30 to 600
     // samples but some lane of the 64 nearly every sample, so that work runs
@@ -442,8 +442,8 @@ struct SweepProg {
     //
     // A lone wavefront pays an issue slot per instruction of any kind, so fewer
     // scalar instructions and branches a sample count there: the Rossler diagram
-    // of 1000 points 28.9 -> 21.1 ms with the pairs, BASINS basins of 200^2
-    // 73.5 -> 57.9 ms.  The pending slots: Lorenz peak map 88.8 -> 86.2 ms at
+    // of 1000 points 28.9 -> 21.1 ms a call with the pairs (20.6 with the slots),
+    // BASINS basins of 200^2 73.5 -> 57.9 ms.  The pending slots: Lorenz peak map 88.8 -> 86.2 ms at
     // 1024^2 points and (sweep alone) 8.1 -> 6.9 ms at 200^2, basins 93.1 ->
     // 91.6 ms at 1024^2; full grids are bound by FP64 issue.  Chameleon's long
     // steps leave them nothing to gain (31.2 -> 31.3 ms at 300^2).
@@ -514,8 +514,8 @@ struct SweepProg {
     // m, vb and tb on lanes n; m and n are disjoint and, as ballots, hold active
     // lanes only.  Values alone are moved under the masks in exec, which then
     // gets back the lanes it had; with times the selects cost no more than that
-    // (1-D Rossler diagram 20.8 -> 20.0 ms, Chameleon peak map of 300^2 points
-    // 31.3 -> 30.7; values only, 1024^2 Lorenz map: selects 1 to 2 % slower).
+    // (1-D Rossler diagram 20.8 -> 20.6 ms, Chameleon peak map of 300^2 points
+    // 31.3 ms both ways; values only, 1024^2 Lorenz map: selects 1 to 2 % slower).
     __device__ __forceinline__ static void to_slots(double& v, int& t, double va, int ta, unsigned long long m,
                                                     double vb, int tb, unsigned long long n)
     {

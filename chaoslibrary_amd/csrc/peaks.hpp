@@ -75,32 +75,6 @@ struct PeakDetector {
         p = cur;
         return emit;
     }
-
-    // feed() for t >= 2 (c = t - 1) without branches: the state machine as
-    // lane predicates, so the hot record loop carries no divergent control
-    // flow.  Same transitions as feed():
-    //   plateau scan or fresh candidate ("act") emits iff d[c]-d[c+1] > 1e-13;
-    //   it stays / becomes a plateau iff the step is flat within 1e-13;
-    //   skip follows an emit or a rejected plateau.
-    __device__ __forceinline__ bool feed_body(int c, double cur, double& val, int& time)
-    {
-        const double dnx = cur - p;
-        const bool c1 = dn > 1e-13;
-        const bool c2 = dnx <= 0.0;
-        const bool c3 = dnx < -1e-13;
-        const bool cand = !plat && !skip && c1 && c2;
-        const bool act = plat || cand;
-        const bool emit = act && c3;
-        const bool flat = c2 && !c3;
-        val = p;
-        time = plat ? (pstart + c) >> 1 : c;
-        pstart = cand && flat ? c : pstart;
-        skip = (plat && !flat) || (cand && c3);
-        plat = act && flat;
-        dn = dnx;
-        p = cur;
-        return emit;
-    }
 };
 
 // Lane mask <-> lane predicate: a compare written straight into a wave mask,
@@ -128,7 +102,7 @@ struct PeakMasks {
         unsigned long long opened;  // lanes that begin a plateau at c
     };
 
-    // PeakDetector::feed_body for every lane (t >= 2).  skip is kept only
+    // PeakDetector::feed for every lane (t >= 2).  skip is kept only
     // where it matters, after a plateau that rose again: after a peak
     // dnx < -1e-13, so the next index fails its own rising test.  So with
     // no plateau open and nothing skipped (quiet), a sample finds no peak and
@@ -239,9 +213,11 @@ struct PeakEntry {
 
 constexpr int kChunk = 256;  // entries per chunk (4 KiB)
 
-// Pool of fixed-size chunks handed out to waves by an atomic head.  Each
-// wave appends its lanes' peaks in time order with one ballot + mbcnt per
-// sample that produced any peak, so a chunk holds one wave's entries densely.
+// Pool of fixed-size chunks handed out to waves by an atomic head.  A wave
+// appends the peaks that wait in its lanes' slots together, with one mbcnt prefix
+// over their mask, so a chunk holds one wave's entries densely: those of a lane
+// in time order, with consecutive sequence numbers (the scatter relies on that),
+// those of different lanes in no order.
 // The bookkeeping sits in one array meta[2 * nchunks + 2] (owner, fill,
 // head, overflow), so a sweep loop holds one pointer for it, not four.
 struct PeakPool {

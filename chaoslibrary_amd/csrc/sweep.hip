@@ -69,7 +69,7 @@ void launch_sweep(CallCtx& ctx, int system, int writableVar, int kind, const Swe
     // wavefronts) runs them one per CU in 64-thread blocks, so that a
     // latency-bound wavefront does not share its CU's scalar unit and
     // instruction issue with three others: 31.9 -> 28.3 ms for that
-    // sweep (20.3 ms with the sample pairs of SweepProg::body).
+    // sweep (20.1 ms with the sample pairs and slots of SweepProg::body).
     // (Grids of a few wavefronts per CU gained nothing and sometimes lost.)
     // The basins epilogue's moments need the 256-thread blocks.
     const bool spread = A.zsum == nullptr &&

@@ -91,7 +91,8 @@ typedef struct chaos_options {
     int device_buffers;     /* compute outputs are device pointers           */
     void* stream;           /* hipStream_t to use; NULL = library stream     */
     int min_pts;            /* CONFIG basins DBSCAN minPts; default 20       */
-    int block;              /* threads per block (0 = tuned default)         */
+    int block;              /* exponent maps: threads per block, a multiple of
+                               64 up to 256 (0 = tuned default)              */
     chaos_stats* stats;     /* optional timing/work report                   */
     int output;             /* map files (2-D outputs): CHAOS_OUT_CSV (default,
                                0 counts as CSV) and/or CHAOS_OUT_BINARY, a
