@@ -77,11 +77,14 @@ __device__ __forceinline__ void legacy_advance(double (&T)[K][System<SYS>::NX], 
 #pragma unroll
     for (int k = 0; k < K; ++k) go[k] = wave_mask(!legacy_bad(T[k][0], A.maxValue));
     for (; left != 0; --left) {
+        unsigned long long any = 0ull;  // lanes with a trajectory that still goes
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             if (lane_bit(go[k])) System<SYS>::step(T[k], a, A.sc);
             if (outside(k) & go[k]) go[k] &= ~wave_mask(legacy_bad(T[k][0], A.maxValue));
+            any |= go[k];
         }
+        if (any == 0ull) return;
     }
 }
 

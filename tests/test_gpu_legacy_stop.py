@@ -38,3 +38,23 @@ def test_exponent_early_stop_matches_oracle(chaos, oracle, sweep_ic, max_value):
     want = oracle.legacy_lle(oracle.SYS["lorenz_rk4"], 0, 1 if sweep_ic else 0, 1, 3.0, 0.1, 130, 0.01, 1e-6, IC, rg,
                              idx, max_value, 1.0, VALUES, 4)
     assert np.allclose(got, want, rtol=1e-10, atol=1e-12, equal_nan=True)
+
+
+# Runs that stop everywhere (a bound that nothing passes, orbits that overflow)
+# end early, after the transient's first step or in the middle of a window.
+@pytest.mark.parametrize("max_value,nt", [(-1.0, 0.5), (0.5, 0.5), (0.0, 2.0)])
+@pytest.mark.parametrize("n", [3, 130])
+def test_all_trajectories_stopped_matches_oracle(chaos, oracle, max_value, nt, n):
+    print(f"legacy, all stopped maxValue={max_value} NT={nt} n={n}", flush=True)
+    # maxValue 0 stops at NaN / inf only: steps of 0.5 make every orbit overflow
+    h, rg = (0.5, [20.0, 40.0]) if max_value == 0.0 else (0.01, [20.0, 40.0])
+    got = chaos.legacy_ls(40 * nt, nt, n, h, 1e-6, IC, rg, [1], 20 * h, VALUES, dims=1, maxValue=max_value,
+                          system="lorenz_rk4", seed=4)
+    want = oracle.legacy_ls(oracle.SYS["lorenz_rk4"], 0, 1, 40 * nt, nt, n, h, 1e-6, IC, rg, [1], max_value, 20 * h,
+                            VALUES, 4)
+    assert np.allclose(got, want, rtol=1e-10, atol=1e-12, equal_nan=True)
+    got = chaos.legacy_lle(40 * nt, nt, n, h, 1e-6, IC, rg, [1], 20 * h, VALUES, dims=1, maxValue=max_value,
+                           system="lorenz_rk4", seed=4)
+    want = oracle.legacy_lle(oracle.SYS["lorenz_rk4"], 0, 0, 1, 40 * nt, nt, n, h, 1e-6, IC, rg, [1], max_value,
+                             20 * h, VALUES, 4)
+    assert np.allclose(got, want, rtol=1e-10, atol=1e-12, equal_nan=True)
