@@ -187,14 +187,6 @@ __host__ __device__ inline double pm_exp(double x)
     return ldexp(p, (int)k);
 }
 
-// The atan series keeps its coefficients where the compiler wants them: DAMIR,
-// its one user, has more coefficients than there are SGPRs, and a wavefront alone
-// on its SIMD pays an issue slot for each scalar move that brings one back.
-// DAMIR basins of 8^2 to 100^2 points, horner / plain: 12.9 / 12.5 ms, legacy
-// exponents 19.5 / 18.8; many wavefronts do not notice the moves but the two
-// instructions a step (basins of 600^2 51.3 / 52.2 ms).  The exponential keeps
-// scalar operands: scalar / plain, with this series plain, 12.5 / 12.3 ms on the
-// small grids and 52.2 / 55.7 ms at 600^2.
 __host__ __device__ inline double pm_atan(double x)
 {
     if (x != x) return x;
@@ -205,17 +197,17 @@ __host__ __device__ inline double pm_atan(double x)
     t = t / (1.0 + sqrt(fma(t, t, 1.0)));
     const double z = t * t;
     double p = 0x1.47ae147ae147bp-5;
-    p = fma(p, z, -0x1.642c8590b2164p-5);
-    p = fma(p, z, 0x1.8618618618618p-5);
-    p = fma(p, z, -0x1.af286bca1af28p-5);
-    p = fma(p, z, 0x1.e1e1e1e1e1e1ep-5);
-    p = fma(p, z, -0x1.1111111111111p-4);
-    p = fma(p, z, 0x1.3b13b13b13b14p-4);
-    p = fma(p, z, -0x1.745d1745d1746p-4);
-    p = fma(p, z, 0x1.c71c71c71c71cp-4);
-    p = fma(p, z, -0x1.2492492492492p-3);
-    p = fma(p, z, 0x1.999999999999ap-3);
-    p = fma(p, z, -0x1.5555555555555p-2);
+    p = pm_horner(p, z, -0x1.642c8590b2164p-5);
+    p = pm_horner(p, z, 0x1.8618618618618p-5);
+    p = pm_horner(p, z, -0x1.af286bca1af28p-5);
+    p = pm_horner(p, z, 0x1.e1e1e1e1e1e1ep-5);
+    p = pm_horner(p, z, -0x1.1111111111111p-4);
+    p = pm_horner(p, z, 0x1.3b13b13b13b14p-4);
+    p = pm_horner(p, z, -0x1.745d1745d1746p-4);
+    p = pm_horner(p, z, 0x1.c71c71c71c71cp-4);
+    p = pm_horner(p, z, -0x1.2492492492492p-3);
+    p = pm_horner(p, z, 0x1.999999999999ap-3);
+    p = pm_horner(p, z, -0x1.5555555555555p-2);
     double v = 4.0 * fma(t * z, p, t);
     if (inv) v = (0x1.921fb54442d18p+0 - v) + 0x1.1a62633145c07p-54;
     return x < 0 ? -v : v;
